@@ -84,6 +84,8 @@ _SIGS = {
     "DiffusionProblem_TimeKernel": (i32, [vp, i32, vp, vp, vp, vp, vp, i32, dp]),
     "DiffusionProblem_SetStencilConfig": (i32, [vp, i32, i32, i32, i32]),
     "DiffusionProblem_GetStencilConfig": (i32, [vp, i32, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32)]),
+    "DiffusionProblem_SetTileConfig": (i32, [vp, i32, i32, i32]),
+    "DiffusionProblem_GetTileConfig": (i32, [vp, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32)]),
     "DiffusionProblem_Autotune": (i32, [vp, i32]),
     "DiffusionProblem_StagePass": (i32, [vp, i32, dp, vp, vp, vp, vp, vp, vp]),
     "Initial": (i32, [d, vp, vp]),
@@ -398,6 +400,15 @@ class Problem:
         v, r, n = i32(), i32(), i32()
         lib().DiffusionProblem_GetStencilConfig(self.h, which, C.byref(v), C.byref(r), C.byref(n))
         return v.value, r.value, n.value
+
+    def set_tile(self, K, rows=4, waves=16):
+        """Register-tile passes of the fused path (K = 0: off)."""
+        return lib().DiffusionProblem_SetTileConfig(self.h, K, rows, waves)
+
+    def get_tile(self):
+        k, r, w = i32(), i32(), i32()
+        lib().DiffusionProblem_GetTileConfig(self.h, C.byref(k), C.byref(r), C.byref(w))
+        return k.value, r.value, w.value
 
     def autotune(self, reps=3):
         return lib().DiffusionProblem_Autotune(self.h, reps)

@@ -537,10 +537,75 @@ void fused_fill(ArkMem* A, const StagePlan& SP, StageEntry* T, int kp)
   ef.out = N_VGetDeviceArrayPointer(A->tv2);
 }
 
+// the fused path on register tiles: stages 2..s in passes of equal length,
+// the first of which forms stage 1 and the last of which adds the closing
+// RHS, so that a step is only these launches.  The operands go by value: no
+// stage table, no copy, and no graph, which the few launches would not repay
+// (a pass takes longer than its launch).
+int stages_tile(ArkMem* A, const StagePlan& SP)
+{
+  const int s = SP.s;
+  DiffusionProblem* P = A->fast;
+  hipStream_t st = P->exec->stream;
+  const bool mms = (P->p.kind == DIFFUSION_MMS_DIRICHLET);
+  N_Vector bufs[4] = {A->tv1, A->ycur, A->tv2, A->tv3};
+  N_Vector Yjm1 = nullptr, Yjm2 = nullptr;
+  for (int j = 2, left = ceda::tile_passes(s - 1, P->tile.K); left > 0; left--) {
+    N_Vector fr[4];
+    int nf = 0;
+    for (N_Vector v : bufs)
+      if (v != Yjm1 && v != Yjm2) fr[nf++] = v;
+    const bool last = left == 1;
+    ceda::TileOps o{};
+    o.K = ceda::tile_len(s - j + 1, left);
+    o.first = j == 2;
+    o.rhs = last && !A->fixedstep;
+    o.yn = N_VGetDeviceArrayPointer(A->yn);
+    o.fn = N_VGetDeviceArrayPointer(A->fn);
+    if (o.first) {
+      o.a0 = 1.0;
+      o.a1 = SP.mus1;
+    } else {
+      o.yjm1 = N_VGetDeviceArrayPointer(Yjm1);
+      o.yjm2 = N_VGetDeviceArrayPointer(Yjm2);
+    }
+    for (int m = 0; m < o.K; m++) {
+      for (int k = 0; k < 5; k++) o.c[8 * m + k] = SP.c[5 * (j + m) + k];
+      if (mms) ceda::mms_time_factors(SP.t[j + m], &o.c[8 * m + 5], &o.c[8 * m + 6]);
+    }
+    // the next-to-last stage is only read by a following pass
+    if (!last) o.outA = N_VGetDeviceArrayPointer(fr[0]);
+    o.outB = N_VGetDeviceArrayPointer(fr[1]);
+    if (o.rhs) {
+      if (mms) ceda::mms_time_factors(A->tn + A->h, &o.c[8 * o.K + 5], &o.c[8 * o.K + 6]);
+      o.outF = N_VGetDeviceArrayPointer(fr[0]);
+    }
+    ceda::launch_tile(P, P->tile, o, st);
+    j += o.K;
+    Yjm2 = fr[0];
+    Yjm1 = fr[1];
+  }
+  // Y_s in Yjm1, F(t_n + h, Y_s) in Yjm2: ycur and tv2
+  N_Vector others[2];
+  int no = 0;
+  for (N_Vector v : bufs)
+    if (v != Yjm1 && v != Yjm2) others[no++] = v;
+  A->ycur = Yjm1;
+  A->tv2 = Yjm2;
+  A->tv1 = others[0];
+  A->tv3 = others[1];
+  CEDA_HIP_CHECK(hipGetLastError());
+  const long nrhs = (s - 1) + (A->fixedstep ? 0 : 1);
+  A->nfe += nrhs;
+  P->nrhs += nrhs;
+  return 0;
+}
+
 int stages_fused(ArkMem* A, const StagePlan& SP)
 {
   const int s = SP.s;
   DiffusionProblem* P = A->fast;
+  if (P->tile.K > 0) return stages_tile(A, SP);
   hipStream_t st = P->exec->stream;
   ensure_table(A, A->smax + 2);
   CEDA_HIP_CHECK(hipEventSynchronize(A->tab_ev));  // previous copy consumed h_tab

@@ -423,7 +423,11 @@ struct TuneKey {
     return nx != o.nx ? nx < o.nx : (ny != o.ny ? ny < o.ny : kind < o.kind);
   }
 };
-std::map<TuneKey, std::array<StencilCfg, 3>> g_tune;
+struct TuneResult {
+  StencilCfg cfg[3];
+  TileCfg tile;
+};
+std::map<TuneKey, TuneResult> g_tune;
 std::mutex g_tune_mu;
 
 bool vec_ok(const DiffusionProblem* P, N_Vector v)
@@ -620,6 +624,7 @@ int DiffusionProblem_SetStencilConfig(DiffusionProblem* P, int which, int varian
   if (!P || which < 0 || which > 2 || rows < 1 || rows > 1024 || nt < 0 || nt > (which == 2 ? 3 : 1)) return -1;
   if (which < 2 && (variant < 0 || variant > 1 || rows > 256 || (variant == 0 && nt))) return -1;
   if (which == 2 && (variant < 0 || variant > kMaxPassStages)) return -1;
+  if (which == 2) P->tile = TileCfg();  // an explicit pass shape replaces the tuned tiles
   P->cfg[which].variant = variant;
   P->cfg[which].rows = rows;
   P->cfg[which].nt = nt;
@@ -633,6 +638,24 @@ int DiffusionProblem_GetStencilConfig(const DiffusionProblem* P, int which, int*
   if (variant) *variant = P->cfg[which].variant;
   if (rows) *rows = P->cfg[which].rows;
   if (nt) *nt = P->cfg[which].nt;
+  return 0;
+}
+
+int DiffusionProblem_SetTileConfig(DiffusionProblem* P, int K, int rows, int waves)
+{
+  if (!P) return -1;
+  const TileCfg t{K, rows, waves};
+  if (K != 0 && !tile_ok(P, t, K, 1)) return -1;
+  P->tile = K ? t : TileCfg();
+  return 0;
+}
+
+int DiffusionProblem_GetTileConfig(const DiffusionProblem* P, int* K, int* rows, int* waves)
+{
+  if (!P) return -1;
+  if (K) *K = P->tile.K;
+  if (rows) *rows = P->tile.R;
+  if (waves) *waves = P->tile.nw;
   return 0;
 }
 
@@ -677,7 +700,8 @@ int DiffusionProblem_Autotune(DiffusionProblem* P, int reps)
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tune.find(key);
     if (it != g_tune.end()) {
-      for (int k = 0; k < 3; k++) P->cfg[k] = it->second[k];
+      for (int k = 0; k < 3; k++) P->cfg[k] = it->second.cfg[k];
+      P->tile = it->second.tile;
       P->tuned = true;
       return 0;
     }
@@ -753,6 +777,45 @@ int DiffusionProblem_Autotune(DiffusionProblem* P, int reps)
     CEDA_HIP_CHECK(ceda::dev_free(dtab));
   }
   P->cfg[2] = bestp;
+  // register-tile passes, where a stage costs less than the best of the above:
+  // 128^2 1.6 against 2.8 us per stage, 777 x 1001 2.2 against 6.6, 2048^2 12.0
+  // against 14.8 (periodic 8.8 against 16.8); at 4096^2, where the four operand
+  // arrays come from HBM for every pass and the tiles' halos with them, 63
+  // against 39
+  TileCfg bestt;
+  float bestt_ms = std::min(best_stage, bestp_ms) * 0.97f;
+  for (int R : {1, 2, 4})
+    for (int nw : {8, 12, 16})
+      for (int K : {3, 4, 6, 8, 10, 12}) {
+        const TileCfg c{K, R, nw};
+        // the closing RHS of a step takes one halo row more; tiles of mostly
+        // halo are never the fastest
+        if (!tile_ok(P, c, K, 1) || (P->p.ny > R * nw && R * nw < 3 * (K + 1))) continue;
+        TileOps o{};
+        o.yjm1 = buf[0];
+        o.yjm2 = buf[1];
+        o.yn = buf[2];
+        o.fn = buf[3];
+        o.outA = buf[4];
+        o.outB = buf[5];
+        o.K = K;
+        for (int m = 0; m < K; m++) {
+          for (int k = 0; k < 5; k++) o.c[8 * m + k] = hc[k];
+          o.c[8 * m + 6] = 1.0;
+        }
+        launch_tile(P, c, o, s);
+        CEDA_HIP_CHECK(hipEventRecord(e0, s));
+        for (int r = 0; r < reps; r++) launch_tile(P, c, o, s);
+        CEDA_HIP_CHECK(hipEventRecord(e1, s));
+        CEDA_HIP_CHECK(hipEventSynchronize(e1));
+        float ms = 0.0f;
+        CEDA_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+        if (ms / K < bestt_ms) {
+          bestt_ms = ms / K;
+          bestt = c;
+        }
+      }
+  P->tile = bestt;
   CEDA_HIP_CHECK(hipEventDestroy(e0));
   CEDA_HIP_CHECK(hipEventDestroy(e1));
   CEDA_HIP_CHECK(hipStreamSynchronize(s));
@@ -760,7 +823,7 @@ int DiffusionProblem_Autotune(DiffusionProblem* P, int reps)
   CEDA_HIP_CHECK(ceda::dev_free(coef));
   P->tuned = true;
   std::lock_guard<std::mutex> lk(g_tune_mu);
-  g_tune[key] = {P->cfg[0], P->cfg[1], P->cfg[2]};
+  g_tune[key] = TuneResult{{P->cfg[0], P->cfg[1], P->cfg[2]}, P->tile};
   return 0;
 }
 

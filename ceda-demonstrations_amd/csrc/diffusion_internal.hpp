@@ -19,6 +19,12 @@ struct StencilCfg {
   int nt = 0;
 };
 
+// shape of the register-tile passes (stage_tile.hip): up to K stages per pass
+// on tiles of nw wavefronts with R rows each; K = 0: not used
+struct TileCfg {
+  int K = 0, R = 0, nw = 0;
+};
+
 struct LearnedPrec;
 struct MGHierarchy;
 
@@ -44,6 +50,7 @@ struct DiffusionProblem {
   // [0] RHS kernel, [1] fused stage kernel, [2] multi-stage pass (variant =
   // stages per pass K, 0 = single-stage kernels only; rows; nt)
   StencilCfg cfg[3];
+  TileCfg tile;  // the autotuner's register-tile shape, where it beats cfg[2]
   LearnedPrec* learned = nullptr;  // network of LearnedPSolve (not owned)
   double learned_out_scale = 1.0;  // its output scale for this problem (LearnedPSetup)
   MGHierarchy* mg = nullptr;       // multigrid hierarchy of MGPSetup/MGPSolve (owned)
@@ -85,6 +92,26 @@ void launch_rhs_entry(DiffusionProblem* P, const StageEntry* e, hipStream_t s);
 void launch_pass(DiffusionProblem* P, int K, int rows, int nt, const StageEntry* e, hipStream_t s);
 // halo lanes of a K-stage pass (each side of a wavefront strip)
 int pass_halo_lanes(int K, int cpl);
+
+// ---- register-tile passes (stage_tile.hip)
+constexpr int kTileMaxK = 12;  // stages per pass
+// the operands of one pass, by value: K stages with the coefficients
+// c[8m .. 8m+4], time factors c[8m+5], c[8m+6]; first: Y_{j-1} = a0 Y_n +
+// a1 F_n and Y_{j-2} = Y_n instead of reading them; outA (may be null): the
+// next-to-last stage, outB: the last one; rhs: also outF = F(last stage)
+// with the time factors c[8K+5], c[8K+6].  Outputs must not alias inputs.
+struct TileOps {
+  const double *yjm1, *yjm2, *yn, *fn;
+  double *outA, *outB, *outF;
+  double a0, a1;
+  int K, first, rhs, pad;
+  double c[8 * (kTileMaxK + 1)];
+};
+bool tile_ok(const DiffusionProblem* P, const TileCfg& t, int K, int rhs);
+void launch_tile(DiffusionProblem* P, const TileCfg& t, const TileOps& o, hipStream_t s);
+// passes of a loop of n stages and the length of the next one: equal lengths
+inline int tile_passes(int n, int K) { return (n + K - 1) / K; }
+inline int tile_len(int left, int passes) { return (left + passes - 1) / passes; }
 
 // ---- batched super-time-stepping (many independent problems, one launch
 // per pass index) ----

@@ -65,6 +65,14 @@ int DiffusionProblem_SetStencilConfig(DiffusionProblem* prob, int which, int var
                                       int nt);
 int DiffusionProblem_GetStencilConfig(const DiffusionProblem* prob, int which, int* variant,
                                       int* rows, int* nt);
+/* [ext] register-tile passes of the fused path: up to K stages (1..12) per
+   launch on tiles of `waves` wavefronts (1..16) with `rows` rows each (1, 2 or
+   4); K = 0: off, the passes of which = 2 are used.  -1 for other values or a tile with nothing left inside its halo.
+   DiffusionProblem_Autotune chooses them where they are fastest (small and
+   middle-sized grids); an explicit DiffusionProblem_SetStencilConfig of
+   which = 2 switches them off.  Bitwise the same results. */
+int DiffusionProblem_SetTileConfig(DiffusionProblem* prob, int K, int rows, int waves);
+int DiffusionProblem_GetTileConfig(const DiffusionProblem* prob, int* K, int* rows, int* waves);
 /* times every candidate launch shape of the three kernels on scratch buffers
    of the problem's size (reps launches each, HIP events) and keeps the
    fastest; multi-stage passes are enabled only when their time per stage
