@@ -543,6 +543,10 @@ DiffusionProblem* DiffusionProblem_Create(const DiffusionParams* prm, SUNContext
     P->fy[j] = coeff(prm->ky, prm->inhomogeneous, yf) / dy2;
     P->py[j] = coeff(prm->ky, prm->inhomogeneous, (double)j * dy) / dy2;
   }
+  auto constant = [](const std::vector<double>& v) {
+    return std::all_of(v.begin(), v.end(), [&](double x) { return x == v[0]; });
+  };
+  P->constant_faces = constant(P->fx) && constant(P->fy) && constant(P->px) && constant(P->py);
   P->sx.assign(nx, 0.0); P->cx.assign(nx, 0.0); P->ax.assign(nx, 0.0);
   P->sy.assign(ny, 0.0); P->cy.assign(ny, 0.0); P->by.assign(ny, 0.0);
   if (per) {

@@ -44,6 +44,7 @@ struct DiffusionProblem {
   N_Vector diag = nullptr;  // Jacobi inverse diagonal (udata->diag, main.cpp:223)
   double diag_gamma = 0.0;       // the gamma of the last PSetup, which computed diag
   bool diag_gamma_set = false;   // diag was last written by PSetup
+  bool constant_faces = false;   // every face table holds one value (constant coefficients)
   SUNContext ctx = nullptr;
   ceda::Exec* exec = nullptr;
   long nrhs = 0;

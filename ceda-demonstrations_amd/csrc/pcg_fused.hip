@@ -4,36 +4,45 @@
 // multigrid preconditioner.  The algorithm is the integrator's PCG
 // (SUNLinSol_PCG, main.cpp:305; Hestenes-Stiefel with z = M r).
 //
-// With Jacobi (or no preconditioner) an iteration l is two kernels:
-//   k_pcg_dirap:  the residual test of iteration l-1 and
+// An iteration l is two kernels:
+//   k_pcg_dir:    the residual test of iteration l-1 and
 //                 beta = r.z(l-1) / r.z(l-2); the direction
 //                 p_l = z + beta p_{l-1}, formed at the five stencil points
-//                 and stored into the other of two direction buffers;
-//                 Ap = p_l - gamma * J p_l and the partial sums of p_l.Ap
-//   k_pcg_update: alpha = r.z / p.Ap; x += alpha p, r -= alpha Ap,
-//                 z = Dinv r (Dinv formed from the face coefficients, not
-//                 read), and the partial sums of |r|^2 and r.z
-// streaming 32 + 56 = 88 bytes per cell (176 for the separate vector
-// operations).  The scalars never go to the host: every workgroup first
-// sums the previous kernel's per-workgroup partials itself, in one fixed
-// order (every workgroup gets bitwise the same alpha or beta, the value a
-// separate one-workgroup combine would give), and the residual test is
-// recorded in a device status word (running, converged at iteration l,
-// non-finite) that every later kernel reads first, returning at once when
-// the solve has ended.  The host enqueues iterations in batches and reads the
-// status once per batch (after a one-workgroup kernel has tested the batch's
-// last iteration): the iteration count, x and the statistics are those of a
-// test after every iteration, and a NaN or infinity stops the solve with an
-// error instead of running to the cap.  The arithmetic of every value is the
-// one of the separate vector operations; only the reductions' summation
-// order differs from them (deterministic, not bitwise equal), which is why
-// this path is an option of the integrator (ARKodeSetDiffusionFastPCG) and
-// the N_Vector PCG stays the reference.
+//                 and stored into the other of two direction buffers; and
+//                 the partial sums of p_l.Ap with Ap = p_l - gamma * J p_l
+//   k_pcg_update: alpha = r.z / p.Ap; x += alpha p, r -= alpha Ap with Ap
+//                 formed again from p_l, and the partial sums of |r|^2, r.z
+// Ap is never stored: the update kernel reads p_l anyway, and its neighbours
+// come from L2.  Nor is z where it is cheap to form: without preconditioner
+// z = r, and with the Jacobi diagonal of constant coefficients z = r times
+// one number.  So an iteration streams 24 + 40 = 64 bytes per cell (88 with z
+// and Ap stored, 176 for the separate vector operations).  With variable
+// coefficients z = r / diag is stored by the update (the eight divisions per
+// pair of cells of forming it at the stencil's points cost more), and a
+// preconditioner given as a callback (multigrid, the learned network) has its
+// z = M r enqueued on the same stream after the update, and k_pcg_dot sums
+// r.z for the next iteration's test and beta.
 //
-// With a preconditioner given as a callback (multigrid, the learned
-// network), the update leaves z alone, the callback's z = M r is enqueued on
-// the same stream after it, and k_pcg_dot sums r.z for the next iteration's
-// test and beta: the scalars stay on the device there too.
+// The scalars never go to the host: every workgroup first sums the previous
+// kernel's per-workgroup partials itself, in one fixed order (every workgroup
+// gets bitwise the same alpha or beta), while its first cells' operands are
+// already being loaded; the residual test is recorded in a device status word
+// (running, converged at iteration l, non-finite) that every later kernel
+// reads first, returning at once when the solve has ended.  The host enqueues
+// iterations in batches, of the previous solve's length at first, and reads
+// the status once per batch (after a one-workgroup kernel has tested the
+// batch's last iteration and written the state to host memory): the iteration
+// count, x and the statistics are those of a test after every iteration, and a
+// NaN or infinity stops the solve with an error instead of running to the cap.
+// The arithmetic of every value is the one of the separate vector operations;
+// only the reductions' summation order differs from them (deterministic, not
+// bitwise equal), which is why this path is an option of the integrator
+// (ARKodeSetDiffusionFastPCG) and the N_Vector PCG stays the reference.
+//
+// Kernel time per iteration with Jacobi: 2048^2 48.3 us, 5.6 TB/s (63.7 us with
+// z and Ap stored); 500 x 480 10.7 us (15.7 us with 938 workgroups, each
+// summing as many partials by LDS shuffles before its first load), which is
+// two kernels' start, partial sums and tail.
 #include <algorithm>
 #include <cmath>
 
@@ -49,16 +58,40 @@ namespace {
 
 constexpr int kPcgBlocks = 1024;   // workgroups of the reduction kernels
 constexpr int kPcgBatchMax = 32;   // iterations enqueued between host checks
+constexpr int kPcgBulkMax = 128;   // the same within the predicted count
+constexpr int kPcgTail = 8;        // iterations between host checks past the predicted count
 constexpr int kPcgChunk = 4;       // callback preconditioner: iterations between host waits in the bulk
 // workspace layout (doubles): partials of p.Ap, of (|r|^2, r.z), of r.z
 // (callback preconditioner), then the solve state
 constexpr int kOffA = 0, kOffB = kPcgBlocks, kOffC = 3 * kPcgBlocks, kOffState = 4 * kPcgBlocks;
-constexpr int kWsDoubles = kOffState + 8;
+constexpr int kStateDoubles = 8;
+constexpr int kWsDoubles = kOffState + kStateDoubles;
 
 // solve state in device memory (doubles): r.z of the current iteration in
 // slot l & 1, the status word, the iteration it was set at, the last |r|^2
 enum { kRz0 = 0, kRz1 = 1, kStatus = 2, kIter = 3, kRr = 4, kDelta = 5 };
 enum { kRunning = 0, kConverged = 1, kNonFinite = 2 };
+
+// x of the lanes `CTRL` (DPP) rows or lanes below; zero where there is none
+template <int CTRL, int ROWS>
+__device__ inline double dpp_or_zero(double x)
+{
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, ROWS, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+// the wavefront's sum, in every lane (row scans of 16 lanes, then the rows)
+__device__ inline double wave_sum(double v)
+{
+  v += dpp_or_zero<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+  v += dpp_or_zero<0x112, 0xf>(v);
+  v += dpp_or_zero<0x114, 0xf>(v);
+  v += dpp_or_zero<0x118, 0xf>(v);
+  v += dpp_or_zero<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v += dpp_or_zero<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), kWave - 1),
+                          __builtin_amdgcn_readlane(__double2loint(v), kWave - 1));
+}
 
 // workgroup sum of NACC accumulators into partials[blockIdx.x * NACC + a]
 template <int NACC>
@@ -68,9 +101,7 @@ __device__ inline void block_sums(double (&acc)[NACC], double* __restrict__ part
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
 #pragma unroll
   for (int a = 0; a < NACC; a++) {
-    double v = acc[a];
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+    const double v = wave_sum(acc[a]);
     if (lane == 0) s[wave][a] = v;
   }
   __syncthreads();
@@ -82,76 +113,39 @@ __device__ inline void block_sums(double (&acc)[NACC], double* __restrict__ part
   }
 }
 
-// the sum of accumulator a over nblocks per-workgroup partials, returned to
-// every thread of the workgroup: thread t adds partials t, t + 256, ... in
-// order, then the wavefront butterfly, then the four wavefront sums in order
-// (every workgroup gets bitwise the same value)
-__device__ inline double sum_partials(const double* __restrict__ partials, int nblocks, int nacc, int a)
+// the sums of NACC accumulators over nblocks per-workgroup partials, returned
+// to every thread of the workgroup: thread t adds partials t, t + 256, ... in
+// order, then the wavefront sum, then the four wavefront sums in order (every
+// workgroup gets bitwise the same values).  TAG: calls of one kernel have
+// LDS words of their own.
+template <int NACC, int TAG>
+__device__ inline void sum_partials(const double* __restrict__ partials, int nblocks, double (&out)[NACC])
 {
-  __shared__ double s[kBlock / kWave];
+  __shared__ double s[kBlock / kWave][NACC];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  double v = 0.0;
-  for (int b = threadIdx.x; b < nblocks; b += kBlock) v += partials[(int64_t)b * nacc + a];
+  double v[NACC] = {};
+  for (int b = threadIdx.x; b < nblocks; b += kBlock)
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-  if (lane == 0) s[wave] = v;
+    for (int a = 0; a < NACC; a++) v[a] += partials[(int64_t)b * NACC + a];
+#pragma unroll
+  for (int a = 0; a < NACC; a++) {
+    const double t = wave_sum(v[a]);
+    if (lane == 0) s[wave][a] = t;
+  }
   __syncthreads();
-  double t = s[0];
 #pragma unroll
-  for (int w = 1; w < kBlock / kWave; w++) t += s[w];
-  __syncthreads();  // s is reused by the next call
-  return t;
+  for (int a = 0; a < NACC; a++) {
+    out[a] = s[0][a];
+#pragma unroll
+    for (int w = 1; w < kBlock / kWave; w++) out[a] += s[w][a];
+  }
 }
-
-// a grid-stride walk over the cells that keeps (i, j) without a division
-// per cell: one division per thread for the start and the stride
-// XCD-aware (as xcd_pairs): when the grid is a multiple of 8, workgroup b
-// walks the (b % 8)-th of 8 contiguous ranges of cells, so that a cell's
-// rows above and below are read by the same XCD at about the same time
-struct CellWalk {
-  int64_t k, i, j, n, nx, step, di, dj;
-  __device__ CellWalk(int64_t n_, int64_t nx_) : n(n_), nx(nx_)
-  {
-    const unsigned G = gridDim.x, b = blockIdx.x;
-    const int parts = (G % 8 == 0) ? 8 : 1;
-    const int64_t per = (n_ + parts - 1) / parts;
-    const int part = (int)(b % parts);
-    k = part * per + (int64_t)(b / parts) * kBlock + threadIdx.x;
-    n = min(n_, (part + 1) * per);
-    j = k / nx;
-    i = k - j * nx;
-    step = (int64_t)(G / parts) * kBlock;
-    dj = step / nx;
-    di = step - dj * nx;
-  }
-  __device__ bool valid() const { return k < n; }
-  __device__ void next()
-  {
-    k += step;
-    i += di;
-    j += dj;
-    if (i >= nx) {
-      i -= nx;
-      j++;
-    }
-  }
-};
 
 __device__ inline bool solve_ended(const double* __restrict__ st) { return st[kStatus] != kRunning; }
 
-// alpha = rz / p.Ap with p.Ap from the stencil kernel's partials (parts_a), then
-// x += alpha p, r -= alpha Ap and
-// mode 0: no preconditioner (z = r), 1: Jacobi (z = dinv r), 2: z computed
-// elsewhere (only x and r are updated; acc[1] = 0).  wl2: the residual norm
-// is the weighted one, sum (r w)^2, else sum r^2.  rz comes from the state
-// (slot l & 1) when st is given, else from the argument.
-// With JAC the update kernel forms the Jacobi inverse diagonal itself
-// instead of reading it: dinv = 1 / (1 - gp d), d = -((ax[i] + ax[i+1]) +
-// (ay[j] + ay[j+1])), exactly k_psetup's value for the gamma gp of the last
-// preconditioner setup: 88 bytes per cell and iteration instead of 96.  (Not
-// storing z at all and forming it at the stencil's five points instead
-// saves 16 more bytes, but the eight divisions per pair of cells make the
-// stencil kernel slower than the traffic saved.)
+// Jacobi inverse diagonal from the face coefficients: dinv = 1 / (1 - gp d),
+// d = -((ax[i] + ax[i+1]) + (ay[j] + ay[j+1])), exactly k_psetup's value for
+// the gamma gp of the last preconditioner setup
 struct JacobiDiag {
   const double *ax, *ay;
   double gp;
@@ -160,42 +154,6 @@ __device__ inline double jac_dinv(const JacobiDiag& J, double sxi, double syj)
 {
   const double d = -(sxi + syj);
   return 1.0 / (1.0 - J.gp * d);
-}
-
-// (the cell-wise update; JAC: mode 1 with the inverse diagonal formed from
-// the face coefficients as above)
-template <bool JAC>
-__global__ __launch_bounds__(kBlock) void k_pcg_update(int64_t n, int64_t nx, int nparts,
-                                                       const double* __restrict__ parts_a, double rz_arg,
-                                                       const double* __restrict__ st, int l,
-                                                       const double* __restrict__ p,
-                                                       const double* __restrict__ ap, double* __restrict__ x,
-                                                       double* __restrict__ r, double* __restrict__ z,
-                                                       const double* __restrict__ dinv, JacobiDiag J,
-                                                       const double* __restrict__ w, int mode,
-                                                       double* __restrict__ partials)
-{
-  if (st && solve_ended(st)) return;
-  const double pap = sum_partials(parts_a, nparts, 1, 0);
-  const double rz = st ? st[l & 1] : rz_arg;
-  const double alpha = rz / pap;
-  double acc[2] = {0.0, 0.0};
-  for (CellWalk c(n, nx); c.valid(); c.next()) {
-    const int64_t k = c.k;
-    x[k] = x[k] + alpha * p[k];
-    const double rk = r[k] + (-alpha) * ap[k];
-    r[k] = rk;
-    const double rw = w ? rk * w[k] : rk;
-    acc[0] += rw * rw;
-    if (mode != 2) {
-      double zk = rk;
-      if (JAC) zk = jac_dinv(J, J.ax[c.i] + J.ax[c.i + 1], J.ay[c.j] + J.ay[c.j + 1]) * rk;
-      else if (mode == 1) zk = dinv[k] * rk;
-      z[k] = zk;
-      acc[1] += rk * zk;
-    }
-  }
-  block_sums<2>(acc, partials);
 }
 
 // the residual test of iteration l-1 from k_pcg_update's partials (|r|^2,
@@ -209,13 +167,20 @@ __device__ inline bool test_iteration(int nparts, const double* __restrict__ par
                                       const double* __restrict__ parts_z, double* __restrict__ st, int l,
                                       double* beta)
 {
-  const double rr = sum_partials(parts_b, nparts, 2, 0);
-  const double rznew = parts_z ? sum_partials(parts_z, nparts, 1, 0) : sum_partials(parts_b, nparts, 2, 1);
+  const double rzold = st[(l - 1) & 1], delta = st[kDelta];
+  double b2[2], z1[1];
+  sum_partials<2, 0>(parts_b, nparts, b2);
+  const double rr = b2[0];
+  double rznew = b2[1];
+  if (parts_z) {
+    sum_partials<1, 1>(parts_z, nparts, z1);
+    rznew = z1[0];
+  }
   const double rnorm = sqrt(rr);
-  *beta = rznew / st[(l - 1) & 1];
+  *beta = rznew / rzold;
   int status = kRunning;
   if (!isfinite(rnorm)) status = kNonFinite;
-  else if (rnorm <= st[kDelta]) status = kConverged;
+  else if (rnorm <= delta) status = kConverged;
   else if (!isfinite(*beta)) status = kNonFinite;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     st[kRr] = rr;
@@ -226,234 +191,287 @@ __device__ inline bool test_iteration(int nparts, const double* __restrict__ par
   return status != kRunning;
 }
 
-__global__ __launch_bounds__(kBlock) void k_pcg_dirap(int64_t nx, int64_t ny, const double* __restrict__ fx,
-                                                      const double* __restrict__ fy, int per, double gamma,
-                                                      const double* __restrict__ z,
-                                                      const double* __restrict__ pold, double* __restrict__ pnew,
-                                                      double* __restrict__ ap, int nparts,
-                                                      const double* __restrict__ parts_b,
-                                                      const double* __restrict__ parts_z,
-                                                      double* __restrict__ parts_a, double* __restrict__ st, int l)
-{
-  if (solve_ended(st)) return;
-  double beta = 0.0;
-  if (l > 1 && test_iteration(nparts, parts_b, parts_z, st, l, &beta)) return;
-  // p_l at a cell: the first direction is z itself, already in pold
-  auto pv = [&](int64_t k) { return (l > 1) ? z[k] + beta * pold[k] : pold[k]; };
-  double acc[1] = {0.0};
-  for (CellWalk c(nx * ny, nx); c.valid(); c.next()) {
-    const int64_t k = c.k, i = c.i, j = c.j;
-    double vw, ve, vs, vn;
-    if (per) {
-      vw = pv(j * nx + (i > 0 ? i - 1 : nx - 1));
-      ve = pv(j * nx + (i < nx - 1 ? i + 1 : 0));
-      vs = pv((j > 0 ? j - 1 : ny - 1) * nx + i);
-      vn = pv((j < ny - 1 ? j + 1 : 0) * nx + i);
-    } else {
-      vw = i > 0 ? pv(k - 1) : 0.0;
-      ve = i < nx - 1 ? pv(k + 1) : 0.0;
-      vs = j > 0 ? pv(k - nx) : 0.0;
-      vn = j < ny - 1 ? pv(k + nx) : 0.0;
-    }
-    const double pk = pv(k);
-    if (l > 1) pnew[k] = pk;
-    const double jp = cell(fx[i], fx[i + 1], fy[j], fy[j + 1], pk, vw, ve, vs, vn);
-    const double a = pk + (-gamma) * jp;  // N_VLinearSum(1, p, -gamma, Jp) order
-    ap[k] = a;
-    acc[0] += pk * a;
-  }
-  block_sums<1>(acc, parts_a);
-}
-
-// The same two kernels on pairs of cells (k, k + 1), k even, for an even
-// nx (a pair never straddles a row): 16-byte loads and stores, half the
-// load instructions of the stencil kernel, which reads z and p_{l-1} at the
-// five points.  Every cell value is the one the cell-wise kernels compute;
-// the dot products group their terms by pairs (a thread adds cell 2q, then
-// 2q + 1), so they differ from the cell-wise kernels' sums in the last bits
-// but are as deterministic.
-// XCD-aware walk over [0, npairs): workgroup b runs on XCD b % 8 and, when
-// the grid is a multiple of 8, walks the (b % 8)-th of 8 contiguous ranges,
-// so that the rows above and below a pair are read by the same XCD at about
-// the same time and come from its L2
-struct PairWalk {
-  int64_t q, end, step;
+// The cells in units of W of a row: W = 2 pairs (k, k + 1), k even, with
+// 16-byte accesses where the rows are even (a pair never straddles a row),
+// W = 1 single cells.  XCD-aware grid-stride walk over the units: workgroup b
+// runs on XCD b % 8 and, when the grid is a multiple of 8, walks the
+// (b % 8)-th of 8 contiguous ranges, so that the rows above and below a unit
+// are read by the same XCD at about the same time and come from its L2.  One
+// division per thread.
+struct PcgGrid {
+  int64_t nx, ny;
+  const double *fx, *fy;
+  int64_t dj;  // rows and units a step advances
+  int64_t di;
 };
-__device__ inline PairWalk xcd_pairs(int64_t npairs)
+template <int W>
+struct UnitWalk {
+  int64_t q, end, step, i, j, hn, di, dj;
+  __device__ UnitWalk(const PcgGrid& g)
+  {
+    const int64_t nu = g.nx * g.ny / W;
+    const unsigned G = gridDim.x, b = blockIdx.x;
+    const int parts = (G % 8 == 0) ? 8 : 1;
+    const int64_t per = (nu + parts - 1) / parts;  // (by a constant 1 or 8)
+    const int part = (int)(b % parts);
+    hn = g.nx / W;
+    q = part * per + (int64_t)(b / parts) * kBlock + threadIdx.x;
+    end = min(nu, (part + 1) * per);
+    step = (int64_t)(G / parts) * kBlock;
+    di = g.di;
+    dj = g.dj;
+    j = nu < ((int64_t)1 << 31) ? (int64_t)((unsigned)q / (unsigned)hn) : q / hn;
+    i = q - j * hn;
+  }
+  __device__ bool valid() const { return q < end; }
+  __device__ void next()
+  {
+    q += step;
+    i += di;
+    j += dj;
+    if (i >= hn) {
+      i -= hn;
+      j++;
+    }
+  }
+};
+// (host) the grid's step in rows and units
+template <int W>
+PcgGrid pcg_grid(const DiffusionProblem* P, unsigned blocks)
 {
-  const unsigned G = gridDim.x, b = blockIdx.x;
-  const int parts = (G % 8 == 0) ? 8 : 1;
-  const int64_t per = (npairs + parts - 1) / parts;
-  const int part = (int)(b % parts);
-  PairWalk w;
-  w.q = part * per + (int64_t)(b / parts) * kBlock + threadIdx.x;
-  w.end = min(npairs, (part + 1) * per);
-  w.step = (int64_t)(G / parts) * kBlock;
-  return w;
+  PcgGrid g;
+  g.nx = P->p.nx;
+  g.ny = P->p.ny;
+  g.fx = P->d_fx;
+  g.fy = P->d_fy;
+  const int64_t step = (int64_t)(blocks / (blocks % 8 == 0 ? 8 : 1)) * kBlock, hn = g.nx / W;
+  g.dj = step / hn;
+  g.di = step - g.dj * hn;
+  return g;
 }
 
-__device__ inline double2 ld2(const double* __restrict__ a, int64_t k)
+template <int W>
+__device__ inline void ldw(const double* __restrict__ a, int64_t k, double (&v)[W])
 {
-  return *reinterpret_cast<const double2*>(a + k);
+  if (W == 2) {
+    const double2 t = *reinterpret_cast<const double2*>(a + k);
+    v[0] = t.x;
+    v[W - 1] = t.y;
+  } else v[0] = a[k];
 }
-__device__ inline void st2(double* __restrict__ a, int64_t k, double2 v) { *reinterpret_cast<double2*>(a + k) = v; }
+template <int W>
+__device__ inline void stw(double* __restrict__ a, int64_t k, const double (&v)[W])
+{
+  if (W == 2) *reinterpret_cast<double2*>(a + k) = make_double2(v[0], v[W - 1]);
+  else a[k] = v[0];
+}
+// a vector at a unit and its neighbours (zero outside a Dirichlet domain)
+template <int W>
+struct Five {
+  double c[W], s[W], n[W], w, e;
+};
+template <bool PER, int W>
+__device__ inline void ld_five(const PcgGrid& g, const UnitWalk<W>& u, const double* __restrict__ a, Five<W>& v)
+{
+  const int64_t nx = g.nx, ny = g.ny, i = u.i * W, k = u.q * W;
+  ldw<W>(a, k, v.c);
+  v.w = v.e = 0.0;
+#pragma unroll
+  for (int t = 0; t < W; t++) v.s[t] = v.n[t] = 0.0;
+  if (PER || i > 0) v.w = a[i > 0 ? k - 1 : k + nx - 1];
+  if (PER || i + W < nx) v.e = a[i + W < nx ? k + W : k + W - nx];
+  if (PER || u.j > 0) ldw<W>(a, u.j > 0 ? k - nx : k + (ny - 1) * nx, v.s);
+  if (PER || u.j < ny - 1) ldw<W>(a, u.j < ny - 1 ? k + nx : k - (ny - 1) * nx, v.n);
+}
+// Ap at the unit: p + (-gamma) J p, N_VLinearSum(1, p, -gamma, Jp) order
+template <int W>
+__device__ inline void ap_of(const PcgGrid& g, const UnitWalk<W>& u, double gamma, const Five<W>& p, double (&ap)[W])
+{
+  const int64_t i = u.i * W;
+  const double h0 = g.fy[u.j], h1 = g.fy[u.j + 1];
+  double f[W + 1];
+#pragma unroll
+  for (int t = 0; t <= W; t++) f[t] = g.fx[i + t];
+#pragma unroll
+  for (int t = 0; t < W; t++) {
+    const double west = t > 0 ? p.c[t > 0 ? t - 1 : 0] : p.w, east = t < W - 1 ? p.c[t < W - 1 ? t + 1 : 0] : p.e;
+    ap[t] = p.c[t] + (-gamma) * cell(f[t], f[t + 1], h0, h1, p.c[t], west, east, p.s[t], p.n[t]);
+  }
+}
 
-template <bool PER>
-__global__ __launch_bounds__(kBlock) void k_pcg_dirap_pairs(int64_t nx, int64_t ny, const double* __restrict__ fx,
-                                                            const double* __restrict__ fy, double gamma,
-                                                            const double* __restrict__ z,
-                                                            const double* __restrict__ pold,
-                                                            double* __restrict__ pnew, double* __restrict__ ap,
-                                                            int nparts, const double* __restrict__ parts_b,
-                                                            const double* __restrict__ parts_z,
-                                                            double* __restrict__ parts_a, double* __restrict__ st,
-                                                            int l)
+// where z comes from: stored, r times the constant Jacobi inverse diagonal, r
+enum { kZStored = 0, kZConst = 1, kZNone = 2 };
+
+template <bool PER, int ZS, int W>
+__global__ __launch_bounds__(kBlock) void k_pcg_dir(const PcgGrid g, double gamma, const double* __restrict__ zr,
+                                                    JacobiDiag J, const double* __restrict__ pold,
+                                                    double* __restrict__ pnew, int nparts,
+                                                    const double* __restrict__ parts_b,
+                                                    const double* __restrict__ parts_z,
+                                                    double* __restrict__ parts_a, double* __restrict__ st, int l)
 {
   if (solve_ended(st)) return;
+  const bool first = (l == 1);  // the first direction is z itself, already in pold
+  UnitWalk<W> u(g);
+  Five<W> z = {}, p = {};
+  if (u.valid()) {  // in flight during the partial sums
+    if (!first) ld_five<PER, W>(g, u, zr, z);
+    ld_five<PER, W>(g, u, pold, p);
+  }
+  const double dz = (ZS == kZConst) ? jac_dinv(J, J.ax[0] + J.ax[1], J.ay[0] + J.ay[1]) : 1.0;
   double beta = 0.0;
-  if (l > 1 && test_iteration(nparts, parts_b, parts_z, st, l, &beta)) return;
-  const bool first = (l == 1);
-  auto pv1 = [&](int64_t k) { return first ? pold[k] : z[k] + beta * pold[k]; };
-  auto pv2 = [&](int64_t k) {
-    const double2 pp = ld2(pold, k);
-    if (first) return pp;
-    const double2 zz = ld2(z, k);
-    return make_double2(zz.x + beta * pp.x, zz.y + beta * pp.y);
-  };
-  const double2 zero2 = make_double2(0.0, 0.0);
+  if (!first && test_iteration(nparts, parts_b, parts_z, st, l, &beta)) return;
+  auto dir = [&](double zv, double pv) { return ((ZS == kZConst) ? dz * zv : zv) + beta * pv; };
   double acc[1] = {0.0};
-  // pair q is cells 2q, 2q + 1 of row j = 2q / nx, columns i, i + 1
-  const int64_t hnx = nx >> 1, npairs = (nx * ny) >> 1;
-  const PairWalk wk = xcd_pairs(npairs);
-  const int64_t step = wk.step;
-  int64_t q = wk.q;
-  int64_t j = q / hnx, i2 = q - j * hnx;
-  const int64_t dj = step / hnx, di = step - dj * hnx;
-  for (; q < wk.end; q += step) {
-    const int64_t k = 2 * q, i = 2 * i2;
-    const double2 c = pv2(k);
-    const double w = i > 0 ? pv1(k - 1) : (PER ? pv1(k + nx - 1) : 0.0);
-    const double e = i + 2 < nx ? pv1(k + 2) : (PER ? pv1(k + 2 - nx) : 0.0);
-    const double2 sv = j > 0 ? pv2(k - nx) : (PER ? pv2(k + (ny - 1) * nx) : zero2);
-    const double2 nv = j < ny - 1 ? pv2(k + nx) : (PER ? pv2(k - (ny - 1) * nx) : zero2);
-    if (!first) st2(pnew, k, c);
-    const double fyj = fy[j], fyj1 = fy[j + 1];
-    const double j0 = cell(fx[i], fx[i + 1], fyj, fyj1, c.x, w, c.y, sv.x, nv.x);
-    const double j1 = cell(fx[i + 1], fx[i + 2], fyj, fyj1, c.y, c.x, e, sv.y, nv.y);
-    const double a0 = c.x + (-gamma) * j0;  // N_VLinearSum(1, p, -gamma, Jp) order
-    const double a1 = c.y + (-gamma) * j1;
-    st2(ap, k, make_double2(a0, a1));
-    acc[0] += c.x * a0;
-    acc[0] += c.y * a1;
-    i2 += di;
-    j += dj;
-    if (i2 >= hnx) {
-      i2 -= hnx;
-      j++;
+  while (u.valid()) {
+    if (!first) {
+#pragma unroll
+      for (int t = 0; t < W; t++) {
+        p.c[t] = dir(z.c[t], p.c[t]);
+        p.s[t] = dir(z.s[t], p.s[t]);
+        p.n[t] = dir(z.n[t], p.n[t]);
+      }
+      p.w = dir(z.w, p.w);
+      p.e = dir(z.e, p.e);
+      stw<W>(pnew, u.q * W, p.c);
+    }
+    double ap[W];
+    ap_of<W>(g, u, gamma, p, ap);
+#pragma unroll
+    for (int t = 0; t < W; t++) acc[0] += p.c[t] * ap[t];
+    u.next();
+    if (u.valid()) {
+      if (!first) ld_five<PER, W>(g, u, zr, z);
+      ld_five<PER, W>(g, u, pold, p);
     }
   }
   block_sums<1>(acc, parts_a);
 }
 
-template <bool JAC>
-__global__ __launch_bounds__(kBlock) void k_pcg_update_pairs(int64_t nx, int64_t ny, int nparts,
-                                                             const double* __restrict__ parts_a,
-                                                             const double* __restrict__ st, int l,
-                                                             const double* __restrict__ p,
-                                                             const double* __restrict__ ap, double* __restrict__ x,
-                                                             double* __restrict__ r, double* __restrict__ z,
-                                                             const double* __restrict__ dinv, JacobiDiag J,
-                                                             const double* __restrict__ w, int mode,
-                                                             double* __restrict__ partials)
+// what the update does about z = M r: nothing (a callback does), r.z with the
+// constant Jacobi inverse diagonal or with z = r (not stored), the Jacobi
+// inverse diagonal from the face coefficients or from an array (stored)
+enum { kUpCallback = 0, kUpConst = 1, kUpNone = 2, kUpJacobi = 3, kUpArray = 4 };
+
+// x += alpha p, r -= alpha Ap.  w: the residual norm is the weighted one, sum
+// (r w)^2, else sum r^2.
+template <bool PER, int UP, int W>
+__global__ __launch_bounds__(kBlock) void k_pcg_update(const PcgGrid g, double gamma, int nparts,
+                                                       const double* __restrict__ parts_a,
+                                                       const double* __restrict__ st, int l,
+                                                       const double* __restrict__ p, double* __restrict__ x,
+                                                       double* __restrict__ r, double* __restrict__ z,
+                                                       const double* __restrict__ dinv, JacobiDiag J,
+                                                       const double* __restrict__ w, double* __restrict__ partials)
 {
   if (solve_ended(st)) return;
-  const double pap = sum_partials(parts_a, nparts, 1, 0);
-  const double alpha = st[l & 1] / pap;
+  UnitWalk<W> u(g);
+  Five<W> pv = {};
+  double xv[W] = {}, rv[W] = {};
+  if (u.valid()) {  // in flight during the partial sums
+    ld_five<PER, W>(g, u, p, pv);
+    ldw<W>(x, u.q * W, xv);
+    ldw<W>(r, u.q * W, rv);
+  }
+  const double dz = (UP == kUpConst) ? jac_dinv(J, J.ax[0] + J.ax[1], J.ay[0] + J.ay[1]) : 1.0;
+  const double rz = st[l & 1];
+  double pap[1];
+  sum_partials<1, 0>(parts_a, nparts, pap);
+  const double alpha = rz / pap[0];
   double acc[2] = {0.0, 0.0};
-  const int64_t hnx = nx >> 1, npairs = (nx * ny) >> 1;
-  const PairWalk wk = xcd_pairs(npairs);
-  const int64_t step = wk.step;
-  int64_t q = wk.q;
-  int64_t j = q / hnx, i2 = q - j * hnx;
-  const int64_t dj = step / hnx, di = step - dj * hnx;
-  for (; q < wk.end; q += step) {
-    const int64_t k = 2 * q;
-    const double2 xv = ld2(x, k), pv = ld2(p, k), rv = ld2(r, k), av = ld2(ap, k);
-    st2(x, k, make_double2(xv.x + alpha * pv.x, xv.y + alpha * pv.y));
-    const double r0 = rv.x + (-alpha) * av.x, r1 = rv.y + (-alpha) * av.y;
-    st2(r, k, make_double2(r0, r1));
-    double rw0 = r0, rw1 = r1;
-    if (w) {
-      const double2 wv = ld2(w, k);
-      rw0 = r0 * wv.x;
-      rw1 = r1 * wv.y;
+  while (u.valid()) {
+    const int64_t k = u.q * W, i = u.i * W;
+    double ap[W], zv[W];
+    ap_of<W>(g, u, gamma, pv, ap);
+#pragma unroll
+    for (int t = 0; t < W; t++) {
+      xv[t] = xv[t] + alpha * pv.c[t];
+      rv[t] = rv[t] + (-alpha) * ap[t];
     }
-    acc[0] += rw0 * rw0;
-    acc[0] += rw1 * rw1;
-    if (mode != 2) {  // 2: z is computed elsewhere
-      double z0 = r0, z1 = r1;
-      if (JAC) {
-        const int64_t i = 2 * i2;
-        const double syj = J.ay[j] + J.ay[j + 1];
-        z0 = jac_dinv(J, J.ax[i] + J.ax[i + 1], syj) * r0;
-        z1 = jac_dinv(J, J.ax[i + 1] + J.ax[i + 2], syj) * r1;
-      } else if (mode == 1) {
-        const double2 dv = ld2(dinv, k);
-        z0 = dv.x * r0;
-        z1 = dv.y * r1;
-      }
-      st2(z, k, make_double2(z0, z1));
-      acc[1] += r0 * z0;
-      acc[1] += r1 * z1;
+    stw<W>(x, k, xv);
+    stw<W>(r, k, rv);
+    double wv[W], dv[W];
+    if (w) ldw<W>(w, k, wv);
+    if (UP == kUpArray) ldw<W>(dinv, k, dv);
+    const double syj = (UP == kUpJacobi) ? J.ay[u.j] + J.ay[u.j + 1] : 0.0;
+#pragma unroll
+    for (int t = 0; t < W; t++) {
+      const double rw = w ? rv[t] * wv[t] : rv[t];
+      acc[0] += rw * rw;
+      if (UP == kUpCallback) continue;
+      zv[t] = rv[t];
+      if (UP == kUpConst) zv[t] = dz * rv[t];
+      if (UP == kUpJacobi) zv[t] = jac_dinv(J, J.ax[i + t] + J.ax[i + t + 1], syj) * rv[t];
+      if (UP == kUpArray) zv[t] = dv[t] * rv[t];
+      acc[1] += rv[t] * zv[t];
     }
-    i2 += di;
-    j += dj;
-    if (i2 >= hnx) {
-      i2 -= hnx;
-      j++;
+    if (UP == kUpJacobi || UP == kUpArray) stw<W>(z, k, zv);
+    u.next();
+    if (u.valid()) {
+      ld_five<PER, W>(g, u, p, pv);
+      ldw<W>(x, u.q * W, xv);
+      ldw<W>(r, u.q * W, rv);
     }
   }
   block_sums<2>(acc, partials);
 }
 
+// the state for the host, written to its (pinned) memory
+__device__ inline void state_to_host(const double* __restrict__ st, double* __restrict__ host)
+{
+  __syncthreads();  // the test's own stores
+  if (threadIdx.x < kStateDoubles) host[threadIdx.x] = st[threadIdx.x];
+}
+
 // the residual test of the last iteration of a batch, so that the host sees it
 __global__ __launch_bounds__(kBlock) void k_pcg_check(int nparts, const double* __restrict__ parts_b,
-                                                      const double* __restrict__ parts_z, double* __restrict__ st,
-                                                      int l)
+                                                      const double* __restrict__ parts_z, double* st, int l,
+                                                      double* host)
 {
-  if (solve_ended(st)) return;
-  double beta;
-  test_iteration(nparts, parts_b, parts_z, st, l, &beta);
+  if (!solve_ended(st)) {
+    double beta;
+    test_iteration(nparts, parts_b, parts_z, st, l, &beta);
+  }
+  state_to_host(st, host);
 }
 
 // the residual test alone of iteration l (callback preconditioner: before
 // z = M r is computed for it): converged or non-finite, recorded as
 // test_iteration does; otherwise the state is left for the next iteration's
 // full test (beta needs r.z)
-__global__ __launch_bounds__(kBlock) void k_pcg_rtest(int nparts, const double* __restrict__ parts_b,
-                                                      double* __restrict__ st, int l)
+__global__ __launch_bounds__(kBlock) void k_pcg_rtest(int nparts, const double* __restrict__ parts_b, double* st, int l,
+                                                      double* host)
 {
-  if (solve_ended(st)) return;
-  const double rr = sum_partials(parts_b, nparts, 2, 0);
-  const double rnorm = sqrt(rr);
-  int status = kRunning;
-  if (!isfinite(rnorm)) status = kNonFinite;
-  else if (rnorm <= st[kDelta]) status = kConverged;
-  if (threadIdx.x == 0 && status != kRunning) {
-    st[kRr] = rr;
-    st[kIter] = l;
-    st[kStatus] = status;
+  if (!solve_ended(st)) {
+    double b2[2];
+    sum_partials<2, 0>(parts_b, nparts, b2);
+    const double rnorm = sqrt(b2[0]);
+    int status = kRunning;
+    if (!isfinite(rnorm)) status = kNonFinite;
+    else if (rnorm <= st[kDelta]) status = kConverged;
+    if (threadIdx.x == 0 && status != kRunning) {
+      st[kRr] = b2[0];
+      st[kIter] = l;
+      st[kStatus] = status;
+    }
   }
+  state_to_host(st, host);
 }
 
+template <int W>
 __global__ __launch_bounds__(kBlock) void k_pcg_dot(int64_t n, const double* __restrict__ a,
                                                     const double* __restrict__ b, double* __restrict__ partials,
                                                     const double* __restrict__ st)
 {
   if (st && solve_ended(st)) return;
   double acc[1] = {0.0};
-  for (int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x; k < n; k += (int64_t)gridDim.x * kBlock)
-    acc[0] += a[k] * b[k];
+  for (int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x; k < n / W; k += (int64_t)gridDim.x * kBlock) {
+    double u[W], v[W];
+    ldw<W>(a, k * W, u);
+    ldw<W>(b, k * W, v);
+#pragma unroll
+    for (int t = 0; t < W; t++) acc[0] += u[t] * v[t];
+  }
   block_sums<1>(acc, partials);
 }
 
@@ -469,9 +487,12 @@ __global__ void k_pcg_init(double* __restrict__ st, double rz, double delta)
   }
 }
 
-unsigned blocks_for(int64_t n)
+// two units per thread at least: each workgroup of the next kernel sums all
+// partials, and below 1,024 of them a kernel is as long as its start
+unsigned blocks_for(int64_t units)
 {
-  int64_t g = (n + kBlock - 1) / kBlock;
+  int64_t g = (units + 2 * kBlock - 1) / (2 * kBlock);
+  if (g >= 8) g = (g + 7) / 8 * 8;  // (the XCD ranges of UnitWalk)
   if (g > kPcgBlocks) g = kPcgBlocks;
   return (unsigned)(g < 1 ? 1 : g);
 }
@@ -482,8 +503,47 @@ void ensure_ws(SUNLinearSolver S)
 {
   if (S->d_ws) return;
   CEDA_HIP_CHECK(dev_malloc(&S->d_ws, sizeof(double) * kWsDoubles));
-  CEDA_HIP_CHECK(host_malloc(&S->h_ws, sizeof(double) * kWsDoubles, hipHostMallocDefault));
+  CEDA_HIP_CHECK(host_malloc(&S->h_ws, sizeof(double) * kStateDoubles, hipHostMallocDefault));
   CEDA_HIP_CHECK(dev_malloc(&S->d_p2, sizeof(double) * vlen(S->r)));
+}
+
+}  // namespace
+
+namespace {
+
+struct PcgArgs {
+  hipStream_t s;
+  unsigned g;
+  double gamma;
+  const double* zsrc;  // what k_pcg_dir forms z from
+  double *z, *x, *r, *pa, *pb, *st;
+  const double *pc, *dinv, *w;
+  JacobiDiag J;
+};
+
+// one iteration's two kernels: p_l into pnew (from pold), x and r
+template <bool PER, int W>
+void launch_iteration(const DiffusionProblem* P, const PcgArgs& a, int zs, int up, const double* pold, double* pnew, int it)
+{
+  const PcgGrid g = pcg_grid<W>(P, a.g);
+#define CEDA_DIR(Z)                                                                                              \
+  hipLaunchKernelGGL((k_pcg_dir<PER, Z, W>), dim3(a.g), dim3(kBlock), 0, a.s, g, a.gamma, a.zsrc, a.J, pold, pnew, \
+                     (int)a.g, a.pb, a.pc, a.pa, a.st, it)
+#define CEDA_UP(U)                                                                                               \
+  hipLaunchKernelGGL((k_pcg_update<PER, U, W>), dim3(a.g), dim3(kBlock), 0, a.s, g, a.gamma, (int)a.g, a.pa, a.st, it, \
+                     pnew, a.x, a.r, a.z, a.dinv, a.J, a.w, a.pb)
+  if (zs == kZConst) CEDA_DIR(kZConst);
+  else if (zs == kZNone) CEDA_DIR(kZNone);
+  else CEDA_DIR(kZStored);
+  switch (up) {
+    case kUpCallback: CEDA_UP(kUpCallback); break;
+    case kUpConst: CEDA_UP(kUpConst); break;
+    case kUpNone: CEDA_UP(kUpNone); break;
+    case kUpJacobi: CEDA_UP(kUpJacobi); break;
+    default: CEDA_UP(kUpArray); break;
+  }
+#undef CEDA_DIR
+#undef CEDA_UP
 }
 
 }  // namespace
@@ -494,27 +554,42 @@ int pcg_fused(ArkMem* A, SUNLinearSolver S, DiffusionProblem* P, int pmode, ARKL
   // the solver's vectors' stream (the problem is the integrator's user data
   // and lives on the same context)
   hipStream_t s = vstream(S->r);
-  const int64_t n = P->n, nx = P->p.nx, ny = P->p.ny;
+  const int64_t n = P->n;
   if (vlen(x) != n || vlen(b) != n || vlen(S->r) != n) {
     fprintf(stderr, "[ARKLS ERROR] fused PCG: vector length %lld does not match the problem's %lld cells\n",
             (long long)vlen(x), (long long)n);
     return -1;
   }
-  const int per = (P->p.kind == DIFFUSION_CEDA_PERIODIC) ? 1 : 0;
-  const unsigned g = blocks_for(n);
+  const bool per = P->p.kind == DIFFUSION_CEDA_PERIODIC;
+  // pairs of cells: an even row length (every pair in one row, every pair's
+  // first cell 16-byte aligned)
+  const bool pairs = (P->p.nx % 2 == 0);
+  const unsigned g = blocks_for(pairs ? n / 2 : n);
   ensure_ws(S);
-  double* pa = S->d_ws + kOffA;
-  double* pb = S->d_ws + kOffB;
+  PcgArgs a{};
+  a.s = s;
+  a.g = g;
+  a.gamma = gamma;
+  a.pa = S->d_ws + kOffA;
+  a.pb = S->d_ws + kOffB;
   double* pc = S->d_ws + kOffC;
-  double* st = S->d_ws + kOffState;
-  double* dx = dptr(x);
-  double* dr = dptr(S->r);
-  double* dz = dptr(S->z);
-  double* dp = dptr(S->p);
-  double* dap = dptr(S->Ap);
-  const double* dinv = (pmode == 1) ? dptr(P->diag) : nullptr;
+  a.pc = pmode == 2 ? pc : nullptr;
+  a.st = S->d_ws + kOffState;
+  a.x = dptr(x);
+  a.r = dptr(S->r);
+  a.z = dptr(S->z);
   const bool wl2 = !(A->ls_reltol > 0.0);
-  const double* w = wl2 ? dptr(A->ewt) : nullptr;
+  a.w = wl2 ? dptr(A->ewt) : nullptr;
+  // the Jacobi inverse diagonal formed in the kernels from the gamma of its
+  // last setup (which is what P->diag holds), or P->diag itself
+  const bool jac = (pmode == 1 && P->diag_gamma_set);
+  a.J = JacobiDiag{per ? P->d_px : P->d_fx, per ? P->d_py : P->d_fy, P->diag_gamma};
+  a.dinv = (pmode == 1) ? dptr(P->diag) : nullptr;
+  int zs = kZStored, up = kUpCallback;
+  if (pmode == 0) zs = kZNone, up = kUpNone;
+  else if (jac && P->constant_faces) zs = kZConst, up = kUpConst;
+  else if (pmode == 1) up = jac ? kUpJacobi : kUpArray;
+  a.zsrc = zs == kZStored ? a.z : a.r;
 
   N_VConst(0.0, x);
   N_VScale(1.0, b, S->r);
@@ -533,138 +608,85 @@ int pcg_fused(ArkMem* A, SUNLinearSolver S, DiffusionProblem* P, int pmode, ARKL
     N_VProd(P->diag, S->r, S->z);
   } else N_VScale(1.0, S->r, S->z);
   N_VScale(1.0, S->z, S->p);
-  double rz = N_VDotProd(S->r, S->z);
+  const double rz = N_VDotProd(S->r, S->z);
   if (krylov_nonfinite("fused PCG", "r.z", rz)) return -1;
 
   // Scalars on the device; the host reads the state once per batch.  The
-  // direction of iteration l lives in q[l & 1] (q[1] = S->p holds p_1 = z).
-  // With a preconditioner callback (multigrid, the learned network) an
-  // iteration is the stencil/direction kernel, the update, the callback's
-  // z = M r (enqueued on the same stream) and r.z (k_pcg_dot).  Every kernel
-  // returns at once after convergence, but the callback's own work would
-  // still be spent, so the host enqueues a fraction (A->pcg_bulk, 3/4 by
-  // default) of the previous solve's iteration count without waiting and
-  // then tests each residual (k_pcg_rtest, one wait) before it calls the
-  // preconditioner.
-  double* q[2] = {S->d_p2, dp};
-  // pairs of cells with 16-byte accesses: an even row length (every pair in
-  // one row, every pair's first cell 16-byte aligned)
-  const bool pairs = (nx % 2 == 0);
-  // the Jacobi inverse diagonal formed in the update kernel (from the gamma
-  // of its last setup, which is what P->diag holds)
-  const bool jac = (pmode == 1 && P->diag_gamma_set);
-  const JacobiDiag J{per ? P->d_px : P->d_fx, per ? P->d_py : P->d_fy, P->diag_gamma};
-  hipLaunchKernelGGL(k_pcg_init, dim3(1), dim3(64), 0, s, st, rz, delta);
+  // direction of iteration l lives in q[l & 1] (q[1] = S->p holds p_1 = z,
+  // which iteration 1 only reads).
+  double* q[2] = {S->d_p2, dptr(S->p)};
+  hipLaunchKernelGGL(k_pcg_init, dim3(1), dim3(64), 0, s, a.st, rz, delta);
+  auto iteration = [&](int it) {
+    const double* pold = it == 1 ? q[1] : q[(it - 1) & 1];
+    if (pairs) {
+      if (per) launch_iteration<true, 2>(P, a, zs, up, pold, q[it & 1], it);
+      else launch_iteration<false, 2>(P, a, zs, up, pold, q[it & 1], it);
+    } else {
+      if (per) launch_iteration<true, 1>(P, a, zs, up, pold, q[it & 1], it);
+      else launch_iteration<false, 1>(P, a, zs, up, pold, q[it & 1], it);
+    }
+  };
+  // the solve's end as the state in S->h_ws says it; zlast: z of the
+  // converged iterate was counted
+  auto ended = [&]() -> int {
+    const long iters = (long)S->h_ws[kIter];
+    A->nli += iters;
+    A->njtimes += iters;
+    if (pmode) A->npsolve += iters - 1;  // z of the converged iterate is not computed or used
+    S->last_iters = iters;
+    if ((int)S->h_ws[kStatus] == kNonFinite) {
+      fprintf(stderr, "[ARKLS ERROR] fused PCG: non-finite residual or direction at iteration %ld "
+                      "(|r|^2 = %g); linear solve failed\n", iters, S->h_ws[kRr]);
+      return -1;
+    }
+    return 0;
+  };
   if (pmode == 2) {
+    // Every kernel returns at once after convergence, but the callback's own
+    // work would still be spent, so the host enqueues a fraction
+    // (A->pcg_bulk, 3/4 by default) of the previous solve's iteration count
+    // without waiting and then tests each residual (k_pcg_rtest, one wait)
+    // before it calls the preconditioner.
     const long bulk = (S->last_iters > 4) ? (long)(A->pcg_bulk * (double)S->last_iters) : 0;
     for (int it = 1; it <= S->maxl; it++) {
-      const double* pold = it == 1 ? q[1] : q[(it - 1) & 1];
-      if (pairs) {
-        if (per)
-          hipLaunchKernelGGL(k_pcg_dirap_pairs<true>, dim3(g), dim3(kBlock), 0, s, nx, ny, P->d_fx, P->d_fy,
-                             gamma, dz, pold, q[it & 1], dap, (int)g, pb, pc, pa, st, it);
-        else
-          hipLaunchKernelGGL(k_pcg_dirap_pairs<false>, dim3(g), dim3(kBlock), 0, s, nx, ny, P->d_fx, P->d_fy,
-                             gamma, dz, pold, q[it & 1], dap, (int)g, pb, pc, pa, st, it);
-        hipLaunchKernelGGL(k_pcg_update_pairs<false>, dim3(g), dim3(kBlock), 0, s, nx, ny, (int)g, pa, st, it,
-                           q[it & 1], dap, dx, dr, dz, dinv, J, w, pmode, pb);
-      } else {
-        hipLaunchKernelGGL(k_pcg_dirap, dim3(g), dim3(kBlock), 0, s, nx, ny, P->d_fx, P->d_fy, per, gamma, dz,
-                           pold, q[it & 1], dap, (int)g, pb, pc, pa, st, it);
-        hipLaunchKernelGGL(k_pcg_update<false>, dim3(g), dim3(kBlock), 0, s, n, nx, (int)g, pa, 0.0, st, it,
-                           q[it & 1], dap, dx, dr, dz, dinv, J, w, pmode, pb);
-      }
+      iteration(it);
       // after the bulk, and every kPcgChunk iterations within it, the host
       // waits for the residual test (chunks keep streams that share a
       // hardware queue interleaved)
       if (it > bulk || it % kPcgChunk == 0) {
-        hipLaunchKernelGGL(k_pcg_rtest, dim3(1), dim3(kBlock), 0, s, (int)g, pb, st, it);
-        CEDA_HIP_CHECK(hipMemcpyAsync(S->h_ws, st, sizeof(double) * 8, hipMemcpyDeviceToHost, s));
+        hipLaunchKernelGGL(k_pcg_rtest, dim3(1), dim3(kBlock), 0, s, (int)g, a.pb, a.st, it, S->h_ws);
         CEDA_HIP_CHECK(hipStreamSynchronize(s));
-        const int status = (int)S->h_ws[kStatus];
-        if (status != kRunning) {
-          const long iters = (long)S->h_ws[kIter];
-          A->nli += iters;
-          A->njtimes += iters;
-          A->npsolve += iters - 1;  // z of the converged iterate is not computed
-          S->last_iters = iters;
-          if (status == kNonFinite) {
-            fprintf(stderr, "[ARKLS ERROR] fused PCG: non-finite residual or direction at iteration %ld "
-                            "(|r|^2 = %g); linear solve failed\n", iters, S->h_ws[kRr]);
-            return -1;
-          }
-          return 0;
-        }
+        if ((int)S->h_ws[kStatus] != kRunning) return ended();
       }
       if (ps(t, A->zcur, A->fz, S->r, S->z, gamma, delta, 1, ud)) {
         fprintf(stderr, "[ARKLS ERROR] fused PCG: the preconditioner solve failed at iteration %d\n", it);
         return -1;
       }
-      hipLaunchKernelGGL(k_pcg_dot, dim3(g), dim3(kBlock), 0, s, n, dr, dz, pc, st);
+      if (pairs) hipLaunchKernelGGL(k_pcg_dot<2>, dim3(g), dim3(kBlock), 0, s, n, a.r, a.z, pc, a.st);
+      else hipLaunchKernelGGL(k_pcg_dot<1>, dim3(g), dim3(kBlock), 0, s, n, a.r, a.z, pc, a.st);
     }
-    hipLaunchKernelGGL(k_pcg_check, dim3(1), dim3(kBlock), 0, s, (int)g, pb, pc, st, S->maxl + 1);
-    CEDA_HIP_CHECK(hipMemcpyAsync(S->h_ws, st, sizeof(double) * 8, hipMemcpyDeviceToHost, s));
-    CEDA_HIP_CHECK(hipStreamSynchronize(s));
-    A->nli += S->maxl;
-    A->njtimes += S->maxl;
-    A->npsolve += S->maxl;
-    S->last_iters = S->maxl;
-    return (sqrt(S->h_ws[kRr]) < bnorm) ? 1 : 2;
   }
-
-  int l = 1, batch = 4;
-  while (l <= S->maxl) {
+  // the batches: most of the previous solve's iterations first, a few at a
+  // time after them; doubling ones without a previous solve
+  const long predicted = S->last_iters > 16 ? S->last_iters - S->last_iters / 16 : 0;
+  int batch = 4;
+  for (int l = 1; pmode != 2 && l <= S->maxl;) {
+    if (predicted) batch = l <= predicted ? (int)std::min<long>(predicted - l + 1, kPcgBulkMax) : kPcgTail;
     const int last = std::min(S->maxl, l + batch - 1);
-    for (int it = l; it <= last; it++) {
-      // iteration 1 reads p_1 = z from q[1] and writes nothing
-      const double* pold = it == 1 ? q[1] : q[(it - 1) & 1];
-      if (pairs) {
-        if (per)
-          hipLaunchKernelGGL(k_pcg_dirap_pairs<true>, dim3(g), dim3(kBlock), 0, s, nx, ny, P->d_fx, P->d_fy,
-                             gamma, dz, pold, q[it & 1], dap, (int)g, pb, nullptr, pa, st, it);
-        else
-          hipLaunchKernelGGL(k_pcg_dirap_pairs<false>, dim3(g), dim3(kBlock), 0, s, nx, ny, P->d_fx, P->d_fy,
-                             gamma, dz, pold, q[it & 1], dap, (int)g, pb, nullptr, pa, st, it);
-        if (jac)
-          hipLaunchKernelGGL(k_pcg_update_pairs<true>, dim3(g), dim3(kBlock), 0, s, nx, ny, (int)g, pa, st, it,
-                             q[it & 1], dap, dx, dr, dz, dinv, J, w, pmode, pb);
-        else
-          hipLaunchKernelGGL(k_pcg_update_pairs<false>, dim3(g), dim3(kBlock), 0, s, nx, ny, (int)g, pa, st, it,
-                             q[it & 1], dap, dx, dr, dz, dinv, J, w, pmode, pb);
-      } else {
-        hipLaunchKernelGGL(k_pcg_dirap, dim3(g), dim3(kBlock), 0, s, nx, ny, P->d_fx, P->d_fy, per, gamma, dz,
-                           pold, q[it & 1], dap, (int)g, pb, nullptr, pa, st, it);
-        if (jac)
-          hipLaunchKernelGGL(k_pcg_update<true>, dim3(g), dim3(kBlock), 0, s, n, nx, (int)g, pa, 0.0, st, it,
-                             q[it & 1], dap, dx, dr, dz, dinv, J, w, pmode, pb);
-        else
-          hipLaunchKernelGGL(k_pcg_update<false>, dim3(g), dim3(kBlock), 0, s, n, nx, (int)g, pa, 0.0, st, it,
-                             q[it & 1], dap, dx, dr, dz, dinv, J, w, pmode, pb);
-      }
-    }
-    hipLaunchKernelGGL(k_pcg_check, dim3(1), dim3(kBlock), 0, s, (int)g, pb, nullptr, st, last + 1);
-    CEDA_HIP_CHECK(hipMemcpyAsync(S->h_ws, st, sizeof(double) * 8, hipMemcpyDeviceToHost, s));
+    for (int it = l; it <= last; it++) iteration(it);
+    hipLaunchKernelGGL(k_pcg_check, dim3(1), dim3(kBlock), 0, s, (int)g, a.pb, nullptr, a.st, last + 1, S->h_ws);
     CEDA_HIP_CHECK(hipStreamSynchronize(s));
-    const int status = (int)S->h_ws[kStatus];
-    const long iters = (long)S->h_ws[kIter];  // iterations run in this solve
-    if (status != kRunning) {
-      A->nli += iters;
-      A->njtimes += iters;
-      if (pmode == 1) A->npsolve += iters - 1;  // z of the converged iterate is not used
-      S->last_iters = iters;
-      if (status == kNonFinite) {
-        fprintf(stderr, "[ARKLS ERROR] fused PCG: non-finite residual or direction at iteration %ld "
-                        "(|r|^2 = %g); linear solve failed\n", iters, S->h_ws[kRr]);
-        return -1;
-      }
-      return 0;
-    }
+    if ((int)S->h_ws[kStatus] != kRunning) return ended();
     l = last + 1;
     batch = std::min(2 * batch, kPcgBatchMax);
   }
+  if (pmode == 2) {
+    hipLaunchKernelGGL(k_pcg_check, dim3(1), dim3(kBlock), 0, s, (int)g, a.pb, pc, a.st, S->maxl + 1, S->h_ws);
+    CEDA_HIP_CHECK(hipStreamSynchronize(s));
+  }
   A->nli += S->maxl;
   A->njtimes += S->maxl;
-  if (pmode == 1) A->npsolve += S->maxl;
+  if (pmode) A->npsolve += S->maxl;
   S->last_iters = S->maxl;
   return (sqrt(S->h_ws[kRr]) < bnorm) ? 1 : 2;
 }
