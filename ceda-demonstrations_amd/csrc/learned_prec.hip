@@ -1353,7 +1353,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_init(int n, double idg, const dou
 //   sweep 2  Ap again from the stored p, x += alpha p, r -= alpha Ap, and
 //            r.r and r.z.
 // Eight vector sweeps of HBM per iteration instead of the textbook loop's
-// eleven (ap = A p; alpha; x, r; beta; p = z + beta p).  PAIRS (even n): a
+// eleven (ap = A p; alpha; x, r; beta; p = z + beta p).  For sides over
+// kCgRegSide only (k_cg_solve otherwise).  PAIRS (even n): a
 // thread takes two cells of a row with 16-byte accesses, and the cells west
 // and east of the pair with 8-byte ones.
 __device__ inline double2 cg_ld2(const double* __restrict__ a, int q) { return *reinterpret_cast<const double2*>(a + q); }
@@ -1460,6 +1461,189 @@ __global__ __launch_bounds__(kBlock) void k_cg_iter(int n, double rx, double ry,
   }
   block_sum2(rr, rz, sh);
   if (threadIdx.x == 0) st[blockIdx.x] = CGState{rz, S.bb, rz / S.rz, rr <= tol2 * S.bb ? 1 : 0, S.iters + 1};
+}
+
+// ---- the same solves with a pair's vectors on one CU
+// One workgroup iterates one pair until it converges (or for `iters`
+// iterations), with r in registers throughout.  Up to kCgLdsSide^2 cells x and
+// Ap are in registers too and p in LDS: an iteration touches no memory, and is
+// bound by its three barriers' phases.  Above, p and x stay in memory: each
+// iteration reads and writes p and x once and reads p's five points twice (48
+// bytes per cell instead of 64), and the pairs being solved, one per CU, stay
+// in the 256 MB of last-level cache (2 x 75 MB at 192^2) where k_cg_iter, which
+// advances every pair by one iteration per launch, streams them all from HBM.
+// Cells are units of W (pairs with 16-byte accesses for even n): unit m of a
+// thread is unit m T + tid of the grid.
+// 1,024 pairs, time per iteration: 192^2 257 us, 7.1 TB/s of cache (537 us,
+// 4.5 TB/s, by k_cg_iter), 128^2 45 us (223), 100^2 33 us (140), 64^2 17 us (48);
+// 1,024 pairs of 192^2 to 1e-12 with 490 iterations 178 ms (380).
+constexpr int kCgLdsSide = 128;   // p in LDS: 128 KiB
+constexpr int kCgRegSide = 192;   // r in registers: 36 cells per thread
+constexpr int kCgCellsLds = 16;   // cells per thread, p in LDS
+constexpr int kCgCellsMem = 36;   // cells per thread, p in memory
+
+__device__ inline double cg_wave_sum(double v)  // the wavefront's sum, in every lane
+{
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+  return v;
+}
+// the workgroup's sum, to every thread, wavefronts in order; sh: kWaves words
+// that no wavefront still reads (callers alternate between two)
+template <int T>
+__device__ inline double cg_block_sum(double v, double* sh)
+{
+  constexpr int kWaves = T / kWave;
+  v = cg_wave_sum(v);
+  if ((threadIdx.x & (kWave - 1)) == 0) sh[threadIdx.x / kWave] = v;
+  __syncthreads();
+  double t = sh[0];
+#pragma unroll
+  for (int w = 1; w < kWaves; w++) t += sh[w];
+  return t;
+}
+
+template <int T, int CPT, int W, bool LDS>
+__global__ __launch_bounds__(T) void k_cg_solve(int n, double rx, double ry, double idg, double tol2, int iters,
+                                                double* __restrict__ x, double* __restrict__ r,
+                                                double* __restrict__ p, CGState* __restrict__ st)
+{
+  constexpr int M = CPT / W;  // units per thread
+  constexpr int kFlight = 3;
+  extern __shared__ double pl[];
+  __shared__ double sh[2][T / kWave];
+  CGState S = st[blockIdx.x];
+  if (S.done) return;
+  const int64_t o = (int64_t)blockIdx.x * n * n;
+  double* __restrict__ xs = x + o;
+  double* __restrict__ rs = r + o;
+  double* ps = p + o;
+  const int h = n / W, nu = h * n, di = T % h, dj = T / h, i0 = (int)threadIdx.x % h, j0 = (int)threadIdx.x / h;
+  auto pld = [&](int k, double (&v)[W]) {
+    if (LDS) {
+#pragma unroll
+      for (int t = 0; t < W; t++) v[t] = pl[k + t];
+    } else if (W == 2) {
+      const double2 u = *reinterpret_cast<const double2*>(ps + k);
+      v[0] = u.x;
+      v[W - 1] = u.y;
+    } else v[0] = ps[k];
+  };
+  auto p1 = [&](int k) { return LDS ? pl[k] : ps[k]; };
+  auto pst = [&](int k, const double (&v)[W]) {
+    if (LDS) {
+#pragma unroll
+      for (int t = 0; t < W; t++) pl[k + t] = v[t];
+    } else if (W == 2) *reinterpret_cast<double2*>(ps + k) = make_double2(v[0], v[W - 1]);
+    else ps[k] = v[0];
+  };
+  // f(m, unit, column unit, row) over the thread's units
+  auto each = [&](auto&& f) {
+    int i = i0, j = j0, q0 = (int)threadIdx.x;
+    // opaque: the units' rows, columns and addresses are not to be kept in
+    // registers from one iteration to the next
+    asm volatile("" : "+v"(i), "+v"(j), "+v"(q0));
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+      const int q = m * T + q0;
+      if (q < nu) f(m, q, i, j);
+      i += di;
+      j += dj;
+      if (i >= h) i -= h, j++;
+      // a few units' loads in flight, not all of them (registers)
+      if (m % kFlight == kFlight - 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // (I - rx Dxx - ry Dyy) p at a unit
+  auto apply = [&](int q, int i, int j, double (&c)[W], double (&v)[W]) {
+    const int k = q * W, ic = i * W;
+    double s[W], no[W];
+    pld(k, c);
+    const double w = ic > 0 ? p1(k - 1) : 0.0, e = ic + W < n ? p1(k + W) : 0.0;
+#pragma unroll
+    for (int t = 0; t < W; t++) s[t] = no[t] = 0.0;
+    if (j > 0) pld(k - n, s);
+    if (j < n - 1) pld(k + n, no);
+#pragma unroll
+    for (int t = 0; t < W; t++)
+      v[t] = op5(c[t], t > 0 ? c[t > 0 ? t - 1 : 0] : w, t < W - 1 ? c[t < W - 1 ? t + 1 : 0] : e, s[t], no[t], rx, ry);
+  };
+  double rr[M][W], xr[LDS ? M : 1][W], ap[LDS ? M : 1][W];
+  each([&](int m, int q, int, int) {
+#pragma unroll
+    for (int t = 0; t < W; t++) {
+      rr[m][t] = rs[q * W + t];
+      if (LDS) {
+        xr[LDS ? m : 0][t] = xs[q * W + t];
+        pl[q * W + t] = ps[q * W + t];
+      }
+    }
+  });
+  const int last = S.iters + iters;
+  while (!S.done && S.iters < last) {
+    // p = z + beta p (own cells; every wavefront has left the last sweep that
+    // read p with the sum that ended it)
+    each([&](int m, int q, int, int) {
+      double v[W];
+      pld(q * W, v);
+#pragma unroll
+      for (int t = 0; t < W; t++) v[t] = rr[m][t] * idg + S.beta * v[t];
+      pst(q * W, v);
+    });
+    __syncthreads();
+    double pap = 0.0;
+    each([&](int m, int q, int i, int j) {
+      double c[W], v[W];
+      apply(q, i, j, c, v);
+#pragma unroll
+      for (int t = 0; t < W; t++) {
+        pap += c[t] * v[t];
+        if (LDS) ap[LDS ? m : 0][t] = v[t];
+      }
+    });
+    const double alpha = S.rz / cg_block_sum<T>(pap, sh[0]);
+    double r2 = 0.0;
+    each([&](int m, int q, int i, int j) {
+      double c[W], v[W];
+      if (LDS) {
+        pld(q * W, c);
+#pragma unroll
+        for (int t = 0; t < W; t++) {
+          v[t] = ap[LDS ? m : 0][t];
+          xr[LDS ? m : 0][t] += alpha * c[t];
+        }
+      } else {
+        apply(q, i, j, c, v);
+        if (W == 2) {
+          double2* xp = reinterpret_cast<double2*>(xs + q * W);
+          const double2 xv = *xp;
+          *xp = make_double2(xv.x + alpha * c[0], xv.y + alpha * c[W - 1]);
+        } else xs[q] += alpha * c[0];
+      }
+#pragma unroll
+      for (int t = 0; t < W; t++) {
+        rr[m][t] = rr[m][t] - alpha * v[t];
+        r2 += rr[m][t] * rr[m][t];
+      }
+    });
+    r2 = cg_block_sum<T>(r2, sh[1]);
+    const double rz = r2 * idg;
+    S.beta = rz / S.rz;
+    S.rz = rz;
+    S.done = r2 <= tol2 * S.bb ? 1 : 0;
+    S.iters++;
+  }
+  each([&](int m, int q, int, int) {
+#pragma unroll
+    for (int t = 0; t < W; t++) {
+      rs[q * W + t] = rr[m][t];
+      if (LDS) {
+        xs[q * W + t] = xr[LDS ? m : 0][t];
+        ps[q * W + t] = pl[q * W + t];
+      }
+    }
+  });
+  if (threadIdx.x == 0) st[blockIdx.x] = S;
 }
 
 unsigned grid_for(int64_t n) { return (unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, 8192); }
@@ -2047,6 +2231,38 @@ void adam_step(LearnedPrec* L, double lr)
   lp_pack(L);
 }
 
+// up to `iters` Jacobi-PCG iterations of every pair on one CU each; false
+// where the sides are too large for it (or the LDS is refused)
+template <int T, int CPT, int W, bool LDS>
+bool launch_cg_solve(int nsamp, int n, double rx, double ry, double idg, double tol2, int iters, double* x, double* r,
+                     double* p, CGState* st, hipStream_t s)
+{
+  const size_t lds = LDS ? sizeof(double) * (size_t)n * n : 0;
+  if (lds > 32768) {
+    static const hipError_t allowed = hipFuncSetAttribute(
+        (const void*)k_cg_solve<T, CPT, W, LDS>, hipFuncAttributeMaxDynamicSharedMemorySize, 8 * T * CPT);
+    if (allowed != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+  }
+  hipLaunchKernelGGL((k_cg_solve<T, CPT, W, LDS>), dim3(nsamp), dim3(T), lds, s, n, rx, ry, idg, tol2, iters, x, r, p, st);
+  return true;
+}
+bool cg_solve(int nsamp, int n, double rx, double ry, double idg, double tol2, int iters, double* x, double* r,
+              double* p, CGState* st, hipStream_t s)
+{
+#define CEDA_CG(T, C, L)                                                                                       \
+  return n % 2 == 0 ? launch_cg_solve<T, C, 2, L>(nsamp, n, rx, ry, idg, tol2, iters, x, r, p, st, s)          \
+                    : launch_cg_solve<T, C, 1, L>(nsamp, n, rx, ry, idg, tol2, iters, x, r, p, st, s)
+  if (n * n <= 256 * kCgCellsLds) CEDA_CG(256, kCgCellsLds, true);
+  if (n * n <= 512 * kCgCellsLds) CEDA_CG(512, kCgCellsLds, true);
+  if (n <= kCgLdsSide) CEDA_CG(1024, kCgCellsLds, true);
+  if (n <= kCgRegSide) CEDA_CG(1024, kCgCellsMem, false);
+#undef CEDA_CG
+  return false;
+}
+
 LearnedPrec* lp_create(int nlayer, const int* dil, SUNContext ctx, bool sym)
 {
   LearnedPrec* L = new LearnedPrec();
@@ -2298,8 +2514,10 @@ int LearnedPrec_MakeTrainingSetXY(int nsamp, int n, double ratio_x, double ratio
   const int maxit = 20000;
   int it = 0;
   bool all = false;
+  constexpr int kChunk = 256;  // iterations per launch of the one-CU solves (a launch of bounded length)
   while (!all && it < maxit) {
-    for (int k = 0; k < 50; k++, it++)
+    if (cg_solve(nsamp, n, ratio_x, ratio_y, idg, reltol * reltol, kChunk, e, tmp, p, st, s)) it += kChunk;
+    else for (int k = 0; k < 50; k++, it++)
       if (n % 2 == 0)
         hipLaunchKernelGGL(k_cg_iter<true>, dim3(nsamp), dim3(kBlock), 0, s, n, ratio_x, ratio_y, idg,
                            reltol * reltol, e, tmp, p, p2, st);
