@@ -69,6 +69,14 @@ struct DiffusionBatch {
   int kpass = ceda::kBatchMaxK;
   int layout = ceda::kLayoutAny;  // shared column layout and boundary of the problems
   bool tuned = false;
+  // register tiles (stage_tile.hip), unless the caller chose marching tiles
+  // (tile rows, thin phases, stages per pass) or most cells are in problems too
+  // large for the last-level cache, where the marching pass is faster (4096^2:
+  // 39 against 63 us per stage)
+  bool tiles = false, tiles_ok = true;
+  std::vector<ceda::TileSlot> geo;  // per problem: the constant part of its slots
+  unsigned char *d_stage = nullptr, *h_stage = nullptr;  // a group's slots, tiles, coefficients (h pinned)
+  size_t cap_stage = 0;
   long ngroups = 0, nlaunches = 0;
   // algorithmic HBM bytes of the phase kernels (FP64 cells): stage 1 reads
   // y_n, F_n and writes Y_1 (24 B); a pass of K stages reads Y_{j-1},
@@ -100,12 +108,25 @@ void host_alloc(T** h, size_t n)
   CEDA_HIP_CHECK(ceda::host_malloc(h, sizeof(T) * (n ? n : 1), hipHostMallocDefault));
 }
 
+void free_staging(DiffusionBatch* B);
+// register tiles on (where they can run) or off; the two paths stage differently
+void use_tiles(DiffusionBatch* B, bool on)
+{
+  on = on && B->tiles_ok;
+  if (on == B->tiles) return;
+  CEDA_HIP_CHECK(hipStreamSynchronize(B->ex->stream));
+  free_staging(B);
+  B->cap_slots = B->cap_tiles = B->cap_vblocks = B->cap_tiles_f = 0;
+  B->cap_stage = 0;
+  B->tiles = on;
+}
+
 void free_staging(DiffusionBatch* B)
 {
-  void* ds[] = {B->d_ent, B->d_tiles, B->d_tiles_f, B->d_err, B->d_s, B->d_part, B->d_dsq};
+  void* ds[] = {B->d_ent, B->d_tiles, B->d_tiles_f, B->d_err, B->d_s, B->d_part, B->d_dsq, B->d_stage};
   for (void* p : ds)
     if (p) CEDA_HIP_CHECK(ceda::dev_free(p));
-  void* hs[] = {B->h_ent, B->h_tiles, B->h_tiles_f, B->h_err, B->h_s, B->h_dsq};
+  void* hs[] = {B->h_ent, B->h_tiles, B->h_tiles_f, B->h_err, B->h_s, B->h_dsq, B->h_stage};
   for (void* p : hs)
     if (p) CEDA_HIP_CHECK(ceda::host_free(p));
   B->d_ent = B->h_ent = nullptr;
@@ -114,6 +135,22 @@ void free_staging(DiffusionBatch* B)
   B->d_err = B->h_err = nullptr;
   B->d_s = B->h_s = nullptr;
   B->d_part = B->d_dsq = B->h_dsq = nullptr;
+  B->d_stage = B->h_stage = nullptr;
+}
+
+// a group's staging on register tiles and its error norms
+void ensure_tile_staging(DiffusionBatch* B, size_t bytes, int slots, int vblocks)
+{
+  if (bytes <= B->cap_stage && slots <= B->cap_slots && vblocks <= B->cap_vblocks) return;
+  CEDA_HIP_CHECK(hipStreamSynchronize(B->ex->stream));
+  free_staging(B);
+  B->cap_stage = std::max(bytes, B->cap_stage);
+  B->cap_slots = std::max(slots, B->cap_slots);
+  B->cap_vblocks = std::max(vblocks, B->cap_vblocks);
+  dev_alloc(&B->d_stage, B->cap_stage);
+  host_alloc(&B->h_stage, B->cap_stage);
+  dev_alloc(&B->d_part, B->cap_vblocks);
+  host_alloc(&B->h_dsq, B->cap_slots);
 }
 
 void ensure_staging(DiffusionBatch* B, int slots, int tiles, int vblocks = 0, int tiles_f = 0)
@@ -250,12 +287,9 @@ void autotune_tiles(DiffusionBatch* B)
   B->tuned = true;
 }
 
-// one step group: every active problem plans an attempt, all planned stage
-// loops run together, then every problem finishes its attempt
-int step_group(DiffusionBatch* B, double tout, bool* progress)
+// the active problems' next attempts
+void plan_group(DiffusionBatch* B, double tout, std::vector<int>& planned)
 {
-  *progress = false;
-  std::vector<int> planned;
   for (size_t k = 0; k < B->probs.size(); k++) {
     BProb& b = B->probs[k];
     if (b.done) continue;
@@ -287,12 +321,11 @@ int step_group(DiffusionBatch* B, double tout, bool* progress)
       break;
     }
   }
-  if (planned.empty()) return 0;
-  *progress = true;
-  std::stable_sort(planned.begin(), planned.end(), [&](int a, int c) {
-    return B->probs[a].SP.s > B->probs[c].SP.s;
-  });
-  const bool adaptive = !B->probs[planned[0]].A->fixedstep;
+}
+
+// the planned stage loops on marching tiles, and the error norms into h_dsq
+void run_marching(DiffusionBatch* B, const std::vector<int>& planned, bool adaptive)
+{
   const bool thin = B->thin_rows > 0;
   int ntiles = 0, nvblocks = 0, ntiles_f = 0;
   for (int k : planned) {
@@ -366,6 +399,146 @@ int step_group(DiffusionBatch* B, double tout, bool* progress)
     B->alg_bytes += cells * (24.0 + 48.0 * (passes - 1) + (last_k >= 2 ? 48.0 : 40.0) +
                              (adaptive ? 16.0 + 32.0 : 0.0));
   }
+}
+
+// The planned stage loops on register tiles, and the error norms into h_dsq.
+// The problems (sorted by stage count) run in sub-batches of at most
+// kTileCells cells, each to its end before the next: the six vectors of a
+// sub-batch then stay in the 256 MB last-level cache over its passes, its
+// problems need about the same number of passes, and the host prepares the
+// next one meanwhile.  256 uneven problems to t = 0.06: BATCHFIG.
+constexpr int64_t kTileCells = (int64_t)4 << 20;
+// below this many tiles of 64 rows a pass runs on tiles of 32 rows (own 10
+// rows instead of 42, half the time per tile): the GPU has 256 CUs
+constexpr int kTileThin = 64;
+size_t align256(size_t n) { return (n + 255) / 256 * 256; }
+void run_tiles(DiffusionBatch* B, const std::vector<int>& planned, bool adaptive)
+{
+  const int nslots = (int)planned.size();
+  size_t bytes = 0;
+  int nvblocks = 0;
+  for (int k : planned) {
+    const BProb& b = B->probs[k];
+    const ceda::TileSlot& g = B->geo[k];
+    bytes += sizeof(ceda::TileSlot) + sizeof(ceda::StsErrItem) +
+             sizeof(ceda::TileRef) * (size_t)(ceda::tile_slot_tiles(g, 0) + ceda::tile_slot_tiles(g, 1)) +
+             sizeof(double) * 8 * (size_t)b.SP.s + 5 * 256;
+    nvblocks = std::max(nvblocks, ceda::sts_err_blocks(b.P->n));
+  }
+  ensure_tile_staging(B, bytes, nslots, nvblocks * nslots);
+  hipStream_t s = B->ex->stream;
+  size_t at = 0;
+  for (int q0 = 0; q0 < nslots;) {
+    int q1 = q0;
+    int64_t cells = 0;
+    while (q1 < nslots && (q1 == q0 || cells + B->probs[planned[q1]].P->n <= kTileCells))
+      cells += B->probs[planned[q1++]].P->n;
+    const int ns = q1 - q0;
+    // this sub-batch's part of the staging: slots, error items, tiles (64 and
+    // 32 rows), coefficients
+    int nt[2] = {0, 0}, stages = 0;
+    for (int q = q0; q < q1; q++) {
+      for (int k = 0; k < 2; k++) nt[k] += ceda::tile_slot_tiles(B->geo[planned[q]], k);
+      stages += B->probs[planned[q]].SP.s;
+    }
+    const size_t begin = at, o_err = begin + align256(sizeof(ceda::TileSlot) * (size_t)ns),
+                 o_t0 = o_err + align256(sizeof(ceda::StsErrItem) * (size_t)ns),
+                 o_t1 = o_t0 + align256(sizeof(ceda::TileRef) * (size_t)nt[0]),
+                 o_c = o_t1 + align256(sizeof(ceda::TileRef) * (size_t)nt[1]),
+                 end = o_c + align256(sizeof(double) * 8 * (size_t)stages);
+    auto* slots = reinterpret_cast<ceda::TileSlot*>(B->h_stage + begin);
+    auto* errs = reinterpret_cast<ceda::StsErrItem*>(B->h_stage + o_err);
+    ceda::TileRef* refs[2] = {reinterpret_cast<ceda::TileRef*>(B->h_stage + o_t0),
+                              reinterpret_cast<ceda::TileRef*>(B->h_stage + o_t1)};
+    auto* coef = reinterpret_cast<double*>(B->h_stage + o_c);
+    std::vector<int> tile_end[2] = {std::vector<int>(ns), std::vector<int>(ns)};
+    int t[2] = {0, 0}, vb = 0, c = 0, maxnp = 0;
+    for (int i = 0; i < ns; i++) {
+      const int k = planned[q0 + i];
+      BProb& b = B->probs[k];
+      ArkMem* A = b.A;
+      const int n = b.SP.s - 1;
+      ceda::TileSlot& T = slots[i];
+      T = B->geo[k];
+      T.s = b.SP.s;
+      T.np = ceda::tile_passes(n, ceda::kTileBatchK);
+      T.a1 = b.SP.mus1;
+      T.yn = N_VGetDeviceArrayPointer(A->yn);
+      T.fn = N_VGetDeviceArrayPointer(A->fn);
+      N_Vector bufs[4] = {A->tv1, A->ycur, A->tv2, A->tv3};
+      for (int m = 0; m < 4; m++) T.buf[m] = N_VGetDeviceArrayPointer(bufs[m]);
+      T.coef = reinterpret_cast<double*>(B->d_stage + o_c) + 8 * (size_t)c;
+      const bool mms = !T.per;
+      for (int j = 2; j <= b.SP.s + 1; j++, c++) {  // the stages, then the closing RHS
+        double* e = coef + 8 * (size_t)c;
+        for (int m = 0; m < 8; m++) e[m] = 0.0;
+        if (j <= b.SP.s)
+          for (int m = 0; m < 5; m++) e[m] = b.SP.c[5 * j + m];
+        if (mms) ceda::mms_time_factors(j <= b.SP.s ? b.SP.t[j] : A->tn + A->h, &e[5], &e[6]);
+      }
+      for (int m = 0; m < 2; m++) {
+        const int rbs = (T.ny + T.own[m] - 1) / T.own[m];
+        for (int rb = 0; rb < rbs; rb++)
+          for (int x = 0; x < T.strips; x++) refs[m][t[m]++] = ceda::TileRef{i, (short)x, (short)rb};
+        tile_end[m][i] = t[m];
+      }
+      // the last pass wrote Y_s and, adaptive, F(t_n + h, Y_s) into its pair
+      const int par = (T.np - 1) & 1;
+      A->ycur = bufs[2 * par + 1];
+      A->tv2 = bufs[2 * par];
+      A->tv1 = bufs[2 - 2 * par];
+      A->tv3 = bufs[3 - 2 * par];
+      // the single-problem path's reduction (raw_sts_error_wsqr), bit for bit
+      const int g = ceda::sts_err_blocks(A->n);
+      errs[i] = ceda::StsErrItem{N_VGetDeviceArrayPointer(A->yn), N_VGetDeviceArrayPointer(A->ycur),
+                                 N_VGetDeviceArrayPointer(A->fn), N_VGetDeviceArrayPointer(A->tv2),
+                                 0.4 * A->h, A->rtol, A->atol, A->n, vb, g};
+      vb += g;
+      maxnp = std::max(maxnp, T.np);
+      const double cell = (double)A->n;
+      // bytes per cell: the first pass reads y_n and F_n (16), the others also
+      // the last two stages (32); all but the last write two stages (16), the
+      // last one and, adaptive, the closing RHS; the error norm reads 32
+      B->alg_bytes += cell * (16.0 + 32.0 * (T.np - 1) + 16.0 * (T.np - 1) + (adaptive ? 16.0 + 32.0 : 8.0));
+    }
+    CEDA_HIP_CHECK(hipMemcpyAsync(B->d_stage + begin, B->h_stage + begin, end - begin, hipMemcpyHostToDevice, s));
+    const auto* dslots = reinterpret_cast<const ceda::TileSlot*>(B->d_stage + begin);
+    const ceda::TileRef* drefs[2] = {reinterpret_cast<const ceda::TileRef*>(B->d_stage + o_t0),
+                                     reinterpret_cast<const ceda::TileRef*>(B->d_stage + o_t1)};
+    int active = ns;
+    for (int q = 0; q < maxnp; q++) {
+      while (active > 0 && slots[active - 1].np <= q) active--;
+      const int k = tile_end[0][active - 1] <= kTileThin ? 1 : 0;
+      ceda::launch_tile_batch(dslots, drefs[k], tile_end[k][active - 1], k, q, adaptive ? 1 : 0, s);
+      B->nlaunches++;
+    }
+    if (adaptive) {  // the norms go to host memory
+      ceda::launch_sts_err_batch(reinterpret_cast<const ceda::StsErrItem*>(B->d_stage + o_err), ns, vb, B->d_part,
+                                 B->h_dsq + q0, s);
+      B->nlaunches++;
+    }
+    CEDA_HIP_CHECK(hipGetLastError());
+    at = end;
+    q0 = q1;
+  }
+}
+
+// one step group: every active problem plans an attempt, all planned stage
+// loops run together, then every problem finishes its attempt
+int step_group(DiffusionBatch* B, double tout, bool* progress)
+{
+  std::vector<int> planned;
+  plan_group(B, tout, planned);
+  *progress = !planned.empty();
+  if (planned.empty()) return 0;
+  std::stable_sort(planned.begin(), planned.end(), [&](int a, int c) {
+    return B->probs[a].SP.s > B->probs[c].SP.s;
+  });
+  const bool adaptive = !B->probs[planned[0]].A->fixedstep;
+  if (B->tiles) run_tiles(B, planned, adaptive);
+  else run_marching(B, planned, adaptive);
+  hipStream_t s = B->ex->stream;
+  const int nslots = (int)planned.size();
   CEDA_HIP_CHECK(hipStreamSynchronize(s));
   B->ngroups++;
   for (int q = 0; q < nslots; q++) {
@@ -434,6 +607,26 @@ DiffusionBatch* DiffusionBatch_Create(int nprob, const DiffusionParams* params,
   if (c2 && all_mms) B->layout = ceda::kLayoutC2Mms;
   else if (c2 && all_per) B->layout = ceda::kLayoutC2Per;
   upload_desc(B);
+  int64_t cells = 0, large = 0;
+  for (const BProb& b : B->probs) {
+    ceda::TileSlot g{};
+    const DiffusionProblem* P = b.P;
+    g.fx = P->d_fx;
+    g.fy = P->d_fy;
+    g.sx = P->d_sx;
+    g.sy = P->d_sy;
+    g.cx = P->d_cx;
+    g.cy = P->d_cy;
+    g.nx = (int)P->p.nx;
+    g.ny = (int)P->p.ny;
+    g.per = P->p.kind == DIFFUSION_CEDA_PERIODIC ? 1 : 0;
+    B->tiles_ok = B->tiles_ok && P->p.nx < (1 << 30) && P->p.ny < (1 << 30) && ceda::tile_slot_geometry(g);
+    B->geo.push_back(g);
+    cells += P->n;
+    if (P->n > kTileCells) large += P->n;
+  }
+  B->tiles_ok = B->tiles_ok && 2 * large <= cells;
+  use_tiles(B, true);
   return B;
 }
 
@@ -483,6 +676,7 @@ int DiffusionBatch_SetMaxNumStages(DiffusionBatch* B, int smax)
   CEDA_HIP_CHECK(hipStreamSynchronize(B->ex->stream));
   free_staging(B);
   B->cap_slots = B->cap_tiles = 0;
+  B->cap_stage = 0;
   B->stride = smax + 2;
   return 0;
 }
@@ -505,6 +699,7 @@ int DiffusionBatch_SetTileRows(DiffusionBatch* B, int rows)
 {
   if (!B || rows < 0 || rows > 256) return ARK_ILL_INPUT;
   B->tile_rows = rows;
+  use_tiles(B, rows == 0);
   if (rows > 0) {
     for (BProb& b : B->probs) set_geometry(b, rows);
     upload_desc(B);
@@ -518,6 +713,7 @@ int DiffusionBatch_SetThinPhases(DiffusionBatch* B, int rows, int min_tiles)
   if (!B || rows < 0 || rows > 256 || min_tiles < 1) return ARK_ILL_INPUT;
   B->thin_rows = rows;
   B->thin_tiles = min_tiles;
+  use_tiles(B, false);
   if (B->tuned) upload_desc(B);
   return 0;
 }
@@ -526,6 +722,7 @@ int DiffusionBatch_SetStagesPerPass(DiffusionBatch* B, int kpass)
 {
   if (!B || kpass < 1 || kpass > ceda::kBatchMaxK) return ARK_ILL_INPUT;
   B->kpass = kpass;
+  use_tiles(B, false);
   if (!B->tile_rows) B->tuned = false;
   return 0;
 }
@@ -543,7 +740,7 @@ int DiffusionBatch_Evolve(DiffusionBatch* B, sunrealtype tout)
     b.new_step = true;
     b.err = 0;
   }
-  if (!B->tuned) autotune_tiles(B);
+  if (!B->tiles && !B->tuned) autotune_tiles(B);
   bool progress = true;
   while (progress) {
     const int r = step_group(B, tout, &progress);

@@ -578,8 +578,6 @@ DiffusionProblem* DiffusionProblem_Create(const DiffusionParams* prm, SUNContext
     }
   }
   upload_tables(P);
-  CEDA_HIP_CHECK(ceda::dev_malloc(&P->d_tf, sizeof(double) * 8));
-  CEDA_HIP_CHECK(ceda::host_malloc(&P->h_tf, sizeof(double) * 8, hipHostMallocDefault));
   P->diag = N_VNew_HipNative(P->n, ctx);
   N_VConst(1.0, P->diag);
   P->cfg[0] = StencilCfg{0, 8, 0};
@@ -594,10 +592,7 @@ void DiffusionProblem_Destroy(DiffusionProblem* P)
   CEDA_HIP_CHECK(hipStreamSynchronize(P->exec->stream));
   N_VDestroy(P->diag);
   ceda::mg_destroy(P->mg);
-  double* ds[] = {P->d_tables, P->d_tf};
-  for (double* d : ds)
-    if (d) CEDA_HIP_CHECK(ceda::dev_free(d));
-  if (P->h_tf) CEDA_HIP_CHECK(ceda::host_free(P->h_tf));
+  if (P->d_tables) CEDA_HIP_CHECK(ceda::dev_free(P->d_tables));
   delete P;
 }
 

@@ -39,8 +39,6 @@ struct DiffusionProblem {
   double *d_sx = nullptr, *d_sy = nullptr, *d_cx = nullptr, *d_cy = nullptr;
   double *d_ax = nullptr, *d_by = nullptr;
   double* d_tables = nullptr;  // the one allocation the d_ tables above point into
-  double* d_tf = nullptr;   // device time factors (T1, T2) for the plain RHS
-  double* h_tf = nullptr;   // pinned staging for d_tf
   N_Vector diag = nullptr;  // Jacobi inverse diagonal (udata->diag, main.cpp:223)
   double diag_gamma = 0.0;       // the gamma of the last PSetup, which computed diag
   bool diag_gamma_set = false;   // diag was last written by PSetup
@@ -101,18 +99,47 @@ constexpr int kTileMaxK = 12;  // stages per pass
 // a1 F_n and Y_{j-2} = Y_n instead of reading them; outA (may be null): the
 // next-to-last stage, outB: the last one; rhs: also outF = F(last stage)
 // with the time factors c[8K+5], c[8K+6].  Outputs must not alias inputs.
-struct TileOps {
+struct TileIO {
   const double *yjm1, *yjm2, *yn, *fn;
   double *outA, *outB, *outF;
   double a0, a1;
   int K, first, rhs, pad;
+};
+struct TileOps : TileIO {
   double c[8 * (kTileMaxK + 1)];
 };
 bool tile_ok(const DiffusionProblem* P, const TileCfg& t, int K, int rhs);
 void launch_tile(DiffusionProblem* P, const TileCfg& t, const TileOps& o, hipStream_t s);
 // passes of a loop of n stages and the length of the next one: equal lengths
-inline int tile_passes(int n, int K) { return (n + K - 1) / K; }
-inline int tile_len(int left, int passes) { return (left + passes - 1) / passes; }
+__host__ __device__ inline int tile_passes(int n, int K) { return (n + K - 1) / K; }
+__host__ __device__ inline int tile_len(int left, int passes) { return (left + passes - 1) / passes; }
+
+// the same passes for many problems in one launch.  A slot is one problem's
+// attempt: np passes of up to kTileBatchK stages over its buffers (pass q
+// reads buf[2(1-q%2)], buf[2(1-q%2)+1] = Y_{j-2}, Y_{j-1} and writes the other
+// two: next-to-last stage, last stage; the last pass leaves F(t_n + h, Y_s)
+// in the first of its pair when adaptive)
+constexpr int kTileBatchK = 10;
+constexpr int kTileBatchWaves = 16;
+struct TileSlot {
+  const double *fx, *fy, *sx, *sy, *cx, *cy;
+  const double *yn, *fn;
+  double* buf[4];
+  const double* coef;  // stage j's {c0..c4, T1, T2, -} at coef + 8 (j - 2), then the closing RHS's
+  double a1;           // Y_1 = Y_n + a1 F_n
+  int nx, ny, per, s, np, strips, hl;
+  int own[2], y0[2];   // rows a tile owns and their offset, R = 4 and R = 2
+};
+struct TileRef {
+  int slot;
+  short strip, rb;
+};
+// a slot's geometry (strips, hl, own, y0) from nx, ny, per; false when the
+// problem is too large for TileRef
+bool tile_slot_geometry(TileSlot& t);
+int tile_slot_tiles(const TileSlot& t, int k);  // tiles with R = 4 (k = 0) or R = 2 (k = 1)
+// pass q of the slots whose tiles are listed
+void launch_tile_batch(const TileSlot* slots, const TileRef* tiles, int ntiles, int k, int q, int adaptive, hipStream_t s);
 
 // ---- batched super-time-stepping (many independent problems, one launch
 // per pass index) ----

@@ -55,7 +55,7 @@ __device__ inline double from_east0(double x)
 // 16 wavefronts share a CU's registers: 128 VGPRs each, which R = 4 fills (R = 8
 // with 8 wavefronts was measured: 5 to 30 % slower on every grid, its row
 // tables spill from the scalar registers)
-constexpr int kTileThreads = 16 * kWave;
+constexpr int kTileThreads = kTileBatchWaves * kWave;
 
 // what a lane keeps of the tables for its two columns, and a wavefront of
 // its R rows (scalar registers)
@@ -116,13 +116,13 @@ struct TileGeo {
   const double *fx, *fy, *sx, *sy, *cx, *cy;
   int64_t nx, ny;
   int strips, hl;  // column strips, halo lanes on each side
-  int own, H;      // rows a tile owns, halo rows above and below
+  int own;         // rows a tile owns
   int y0;          // row offset of a tile's first row from its first owned one
 };
 
 // the pass on one tile: K stages with the coefficients sc[8*m .. 8*m+6]
 template <int R, bool PER, bool MMS>
-__device__ __forceinline__ void tile_pass(const TileGeo& g, const TileOps& o, ccdouble* sc, int strip, int rb,
+__device__ __forceinline__ void tile_pass(const TileGeo& g, const TileIO& o, ccdouble* sc, int strip, int rb,
                                           double2* lds, int nw)
 {
   const int lane = threadIdx.x & (kWave - 1);
@@ -312,6 +312,74 @@ __global__ __launch_bounds__(kTileThreads) void k_tile(const TileGeo g, const Ti
   tile_pass<R, PER, MMS>(g, o, (ccdouble*)o.c, strip, rb, tile_lds, (int)(blockDim.x / kWave));
 }
 
+// column strips and owned rows of tiles of `rows` rows with halo H.  A
+// Dirichlet domain no larger than the tile needs no halo: what lies outside is
+// the zero ghosts.
+void tile_shape(int64_t nx, int64_t ny, bool per, int64_t rows, int H, int& strips, int& hl, int& own, int& y0)
+{
+  if (!per && nx <= 2 * kWave) {
+    hl = 0;
+    strips = 1;
+  } else {
+    hl = (H + 1) / 2;
+    const int64_t ow = 2 * (kWave - 2 * hl);
+    strips = (int)((nx + ow - 1) / ow);
+  }
+  if (!per && ny <= rows) {
+    own = (int)ny;
+    y0 = 0;
+  } else {
+    own = (int)(rows - 2 * H);
+    y0 = -H;
+  }
+}
+
+// one tile of pass q of its slot (see TileSlot)
+template <int R>
+__global__ __launch_bounds__(kTileThreads) void k_tile_batch(const TileSlot* __restrict__ slots,
+                                                             const TileRef* __restrict__ tiles, int k, int q,
+                                                             int adaptive)
+{
+  extern __shared__ double2 tile_lds[];
+  const unsigned nb = gridDim.x, b = blockIdx.x;
+  const unsigned bq = nb >> 3, br = nb & 7u, xcd = b & 7u, loc = b >> 3;
+  const TileRef ref = tiles[xcd * bq + (xcd < br ? xcd : br) + loc];  // XCD-aware order
+  const TileSlot& t = slots[ref.slot];
+  TileGeo g;
+  g.fx = t.fx;
+  g.fy = t.fy;
+  g.sx = t.sx;
+  g.sy = t.sy;
+  g.cx = t.cx;
+  g.cy = t.cy;
+  g.nx = t.nx;
+  g.ny = t.ny;
+  g.strips = t.strips;
+  g.hl = t.hl;
+  g.own = t.own[k];
+  g.y0 = t.y0[k];
+  // pass q of np of nearly equal lengths (tile_len: the first ones longer)
+  const int n = t.s - 1, base = n / t.np, rem = n - base * t.np;
+  const int j = 2 + q * base + (q < rem ? q : rem), par = q & 1;
+  const bool last = q == t.np - 1;
+  TileIO o;
+  o.K = base + (q < rem ? 1 : 0);
+  o.first = q == 0;
+  o.rhs = last && adaptive;
+  o.yn = t.yn;
+  o.fn = t.fn;
+  o.a0 = 1.0;
+  o.a1 = t.a1;
+  o.yjm2 = t.buf[2 - 2 * par];
+  o.yjm1 = t.buf[3 - 2 * par];
+  o.outA = last ? nullptr : t.buf[2 * par];
+  o.outB = t.buf[2 * par + 1];
+  o.outF = t.buf[2 * par];
+  ccdouble* sc = (ccdouble*)(t.coef + 8 * (j - 2));
+  if (t.per) tile_pass<R, true, false>(g, o, sc, ref.strip, ref.rb, tile_lds, kTileBatchWaves);
+  else tile_pass<R, false, true>(g, o, sc, ref.strip, ref.rb, tile_lds, kTileBatchWaves);
+}
+
 TileGeo tile_geo(const DiffusionProblem* P, const TileCfg& t, int H)
 {
   TileGeo g;
@@ -323,26 +391,7 @@ TileGeo tile_geo(const DiffusionProblem* P, const TileCfg& t, int H)
   g.cy = P->d_cy;
   g.nx = P->p.nx;
   g.ny = P->p.ny;
-  g.H = H;
-  const bool per = P->p.kind == DIFFUSION_CEDA_PERIODIC;
-  const int64_t rows = (int64_t)t.R * t.nw;
-  // a Dirichlet domain no larger than the tile needs no halo: what lies
-  // outside is the zero ghosts
-  if (!per && P->p.nx <= 2 * kWave) {
-    g.hl = 0;
-    g.strips = 1;
-  } else {
-    g.hl = (H + 1) / 2;
-    const int64_t ow = 2 * (kWave - 2 * g.hl);
-    g.strips = (int)((P->p.nx + ow - 1) / ow);
-  }
-  if (!per && P->p.ny <= rows) {
-    g.own = (int)P->p.ny;
-    g.y0 = 0;
-  } else {
-    g.own = (int)(rows - 2 * H);
-    g.y0 = -H;
-  }
+  tile_shape(g.nx, g.ny, P->p.kind == DIFFUSION_CEDA_PERIODIC, (int64_t)t.R * t.nw, H, g.strips, g.hl, g.own, g.y0);
   return g;
 }
 
@@ -376,6 +425,27 @@ void launch_tile(DiffusionProblem* P, const TileCfg& t, const TileOps& o, hipStr
     default: CEDA_TILE(4) break;
   }
 #undef CEDA_TILE
+}
+
+bool tile_slot_geometry(TileSlot& t)
+{
+  for (int k = 0; k < 2; k++) {
+    tile_shape(t.nx, t.ny, t.per, kTileBatchWaves * (k == 0 ? 4 : 2), kTileBatchK + 1, t.strips, t.hl, t.own[k], t.y0[k]);
+    if (t.strips > 32767 || (t.ny + t.own[k] - 1) / t.own[k] > 32767) return false;
+  }
+  return true;
+}
+
+int tile_slot_tiles(const TileSlot& t, int k) { return t.strips * ((t.ny + t.own[k] - 1) / t.own[k]); }
+
+void launch_tile_batch(const TileSlot* slots, const TileRef* tiles, int ntiles, int k, int q, int adaptive, hipStream_t s)
+{
+  if (ntiles <= 0) return;
+  const size_t lds = sizeof(double2) * 2 * 2 * kWave * kTileBatchWaves;
+  if (k == 0)
+    hipLaunchKernelGGL(k_tile_batch<4>, dim3(ntiles), dim3(kTileThreads), lds, s, slots, tiles, k, q, adaptive);
+  else
+    hipLaunchKernelGGL(k_tile_batch<2>, dim3(ntiles), dim3(kTileThreads), lds, s, slots, tiles, k, q, adaptive);
 }
 
 }  // namespace ceda
