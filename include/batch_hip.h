@@ -34,7 +34,10 @@ int DiffusionBatch_SetController(DiffusionBatch* B, int controller);    /* ARK_A
 int DiffusionBatch_SetMaxNumStages(DiffusionBatch* B, int smax);
 int DiffusionBatch_SetMaxNumSteps(DiffusionBatch* B, long mxsteps);
 int DiffusionBatch_SetFixedStep(DiffusionBatch* B, sunrealtype h);
-/* tile height of the batched kernels: each wavefront tile is `rows` rows of a
+/* The stage loops run on register tiles unless one of the next three is called
+   with other than SetTileRows(B, 0); the results do not depend on it.
+
+   tile height of the marching kernels: each wavefront tile is `rows` rows of a
    124-column strip (62 for odd nx); rows 1..256, 0 = choose per size class by
    the tile autotuner */
 int DiffusionBatch_SetTileRows(DiffusionBatch* B, int rows);
@@ -44,7 +47,7 @@ int DiffusionBatch_SetTileRows(DiffusionBatch* B, int rows);
    marches over more wavefronts); rows 1..256, 0 = never; defaults 12 and
    2048.  The results do not depend on it. */
 int DiffusionBatch_SetThinPhases(DiffusionBatch* B, int rows, int min_tiles);
-/* stages per pass of the batched multi-stage kernel (1..5, default 5): each
+/* stages per pass of the marching multi-stage kernel (1..5, default 5): each
    phase launch advances every active problem by up to this many stages */
 int DiffusionBatch_SetStagesPerPass(DiffusionBatch* B, int kpass);
 /* advance every problem to tout; returns 0, or the first failing problem's
@@ -55,11 +58,13 @@ int DiffusionBatch_GetSolution(DiffusionBatch* B, int p, N_Vector y);
 int DiffusionBatch_GetCurrentTime(DiffusionBatch* B, int p, sunrealtype* t);
 /* same layout as ARKodeGetStatsArray */
 int DiffusionBatch_GetStatsArray(DiffusionBatch* B, int p, long* out, int nout);
-/* step groups and stage-phase launches issued so far */
+/* step groups, and pass and error-norm launches, issued so far */
 int DiffusionBatch_GetNumGroups(DiffusionBatch* B, long* ngroups, long* nlaunches);
-/* algorithmic HBM bytes the phase kernels have moved so far (FP64 cells:
-   24 B per cell for a first stage, 48 for a pass of up to kpass stages, 16
-   for the closing RHS, 32 for the error norm), for roofline accounting */
+/* algorithmic bytes the stage and error-norm kernels have moved so far (FP64
+   cells), for roofline accounting.  Register tiles: 16 B per cell read by the
+   first pass, 48 by each later one, 16 written by each pass (8 by the last one
+   of a fixed step), 32 for the error norm.  Marching tiles: 24 for a first
+   stage, 48 for a pass, 16 for the closing RHS, 32 for the error norm. */
 int DiffusionBatch_GetAlgorithmicBytes(DiffusionBatch* B, double* bytes);
 
 #ifdef __cplusplus
