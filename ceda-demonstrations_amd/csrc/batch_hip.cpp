@@ -624,6 +624,7 @@ DiffusionBatch* DiffusionBatch_Create(int nprob, const DiffusionParams* params,
     g.nx = (int)P->p.nx;
     g.ny = (int)P->p.ny;
     g.per = P->p.kind == DIFFUSION_CEDA_PERIODIC ? 1 : 0;
+    g.cc = P->constant_faces ? 1 : 0;
     B->tiles_ok = B->tiles_ok && P->p.nx < (1 << 30) && P->p.ny < (1 << 30) && ceda::tile_slot_geometry(g);
     B->geo.push_back(g);
     cells += P->n;

@@ -127,7 +127,7 @@ struct TileSlot {
   double* buf[4];
   const double* coef;  // stage j's {c0..c4, T1, T2, -} at coef + 8 (j - 2), then the closing RHS's
   double a1;           // Y_1 = Y_n + a1 F_n
-  int nx, ny, per, s, np, strips, hl;
+  int nx, ny, per, cc, s, np, strips, hl;  // cc: constant coefficients
   int own[2], y0[2];   // rows a tile owns and their offset, R = 4 and R = 2
 };
 struct TileRef {

@@ -17,13 +17,15 @@
 //
 // Against the marching pass (k_pass), which re-forms each row's chain of K
 // dependent stages serially, a stage here is one short burst of 2R
-// independent cells per lane: it is bound by the FP64 issue rate (about 28
-// instructions per cell: 128 x 64 cells of one CU take 1.6 us) or, on small
+// independent cells per lane: it is bound by the FP64 issue rate (about 24
+// instructions per cell: 128 x 64 cells of one CU take 1.3 us) or, on small
 // grids, by the launch, where k_pass is bound by its dependency chains.
 // Per stage, at the best shape of each: 128^2 1.6 us (before: 2.8 us by single
 // stages; a 3-stage k_pass 4.9 us), 777 x 1001 periodic 2.2 us (6.6), 2048^2
 // 12.0 us (14.8).  The adaptive RKC solve at 128^2 to t = 1 (560 steps of 19
-// right-hand sides) went from 49.9 to 29.5 ms.
+// right-hand sides) went from 49.9 to 29.5 ms, and to 27.9 ms with the products
+// of constant coefficients shared between cells (tile_stage_cc), which takes
+// 256 uneven problems in a batch from 593 to 536 ms.
 //
 // Every value is formed by cell(), forcing() and lc5() in their order: the
 // result is bitwise that of the single-stage kernels.
@@ -61,54 +63,102 @@ constexpr int kTileThreads = kTileBatchWaves * kWave;
 // its R rows (scalar registers)
 template <int R>
 struct TileTab {
+  double fx, fy, mdiag;  // constant coefficients: the faces' values and minus the diagonal
   double Dw0, De0, Dw1, De1, sx0, sx1, cx0, cx1;
   double Ds[R], Dn[R], sy[R], cy[R];
   bool in0, in1;  // the columns lie in the domain
   int64_t j;      // the wavefront's first row
 };
 
-// The forcing's factor cx*sy + cy*sx and the centre's coefficient do not change
-// from stage to stage.  Kept in registers they cost 4R VGPRs each, which the
-// R = 4 tiles do not have: there the row's table values pass through an empty
-// asm every stage, so that the compiler forms the products again.
+// The forcing's factor cx*sy + cy*sx does not change from stage to stage.  Kept
+// in registers it costs 4R VGPRs, which the R = 4 tiles do not have: there the
+// row's table values pass through an empty asm every stage, so that the
+// compiler forms the products again.
 constexpr int kHideTab = 4;
 
-// F of the wavefront's rows from Y (S, N: the rows below and above them);
-// MASK: zero outside the domain (the Dirichlet ghosts).  Then lc5 with the
-// stage's coefficients (COMB), the result over prev.
-template <int R, bool MMS, bool MASK, bool COMB>
-__device__ __forceinline__ void tile_stage(const TileTab<R>& t, int64_t ny, const double (&c)[7], double (&prev)[R][2],
+// F of the wavefront's rows from Y (S, N: the rows below and above them), then
+// lc5 with the stage's coefficients (COMB), the result over prev.  Varying
+// coefficients (periodic only)
+template <int R, bool COMB>
+__device__ __forceinline__ void tile_stage(const TileTab<R>& t, const double (&c)[7], double (&prev)[R][2],
                                            const double (&cur)[R][2], const double (&yn)[R][2],
                                            const double (&fn)[R][2], double2 S, double2 N)
 {
-  const double T1 = c[5], T2 = c[6];
 #pragma unroll
   for (int q = 0; q < R; q++) {
     // the rows the neighbouring wavefronts wait for first: 0, R-1, 1, 2, ...
     const int r = q == 0 ? 0 : (q == 1 ? R - 1 : q - 1);
-    if (MASK && (t.j + r < 0 || t.j + r >= ny)) continue;  // a row of ghosts: prev is and stays zero
-    double syj = t.sy[r], cyj = t.cy[r], Ds = t.Ds[r];
-    if (MMS && R >= kHideTab) asm volatile("" : "+s"(syj), "+s"(cyj), "+s"(Ds));
     const double s0 = r > 0 ? cur[r > 0 ? r - 1 : 0][0] : S.x, s1 = r > 0 ? cur[r > 0 ? r - 1 : 0][1] : S.y;
     const double n0 = r < R - 1 ? cur[r < R - 1 ? r + 1 : 0][0] : N.x;
     const double n1 = r < R - 1 ? cur[r < R - 1 ? r + 1 : 0][1] : N.y;
     const double w = from_west0(cur[r][1]), e = from_east0(cur[r][0]);
-    double f0 = cell(t.Dw0, t.De0, Ds, t.Dn[r], cur[r][0], w, cur[r][1], s0, n0);
-    double f1 = cell(t.Dw1, t.De1, Ds, t.Dn[r], cur[r][1], cur[r][0], e, s1, n1);
-    if (MMS) {
-      f0 = f0 + forcing(T1, T2, t.sx0, t.cx0, syj, cyj);
-      f1 = f1 + forcing(T1, T2, t.sx1, t.cx1, syj, cyj);
-    }
+    double f0 = cell(t.Dw0, t.De0, t.Ds[r], t.Dn[r], cur[r][0], w, cur[r][1], s0, n0);
+    double f1 = cell(t.Dw1, t.De1, t.Ds[r], t.Dn[r], cur[r][1], cur[r][0], e, s1, n1);
     if (COMB) {
       f0 = lc5(c, f0, prev[r][0], yn[r][0], cur[r][0], fn[r][0]);
       f1 = lc5(c, f1, prev[r][1], yn[r][1], cur[r][1], fn[r][1]);
     }
-    if (MASK) {
-      f0 = t.in0 ? f0 : 0.0;
-      f1 = t.in1 ? f1 : 0.0;
-    }
     prev[r][0] = f0;
     prev[r][1] = f1;
+  }
+}
+
+// tile_stage where every face coefficient in x is one value and every one in y
+// another (the manufactured problem always).  MASK: zero outside the domain
+// (the Dirichlet ghosts).  The products of a cell with them
+// are formed once and handed to its neighbours, so F takes 3 multiplications
+// and 4 additions instead of 5 and 8, the diagonal being one number.  The terms
+// and their order are cell()'s; its 0 + t, which only turns a -0 into +0, is
+// left out of the stages.
+template <int R, bool MMS, bool MASK, bool COMB>
+__device__ __forceinline__ void tile_stage_cc(const TileTab<R>& t, int64_t ny, const double (&c)[7],
+                                              double (&prev)[R][2], const double (&cur)[R][2],
+                                              const double (&yn)[R][2], const double (&fn)[R][2], double2 S, double2 N)
+{
+  const double T1 = c[5], T2 = c[6];
+  double s0 = t.fy * S.x, s1 = t.fy * S.y;  // fy times the rows below, here and above
+  double m0 = t.fy * cur[0][0], m1 = t.fy * cur[0][1];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const double n0 = t.fy * (r < R - 1 ? cur[r < R - 1 ? r + 1 : 0][0] : N.x);
+    const double n1 = t.fy * (r < R - 1 ? cur[r < R - 1 ? r + 1 : 0][1] : N.y);
+    if (!MASK || (t.j + r >= 0 && t.j + r < ny)) {  // else a row of ghosts: prev is and stays zero
+      double syj = t.sy[r], cyj = t.cy[r];
+      if (MMS && R >= kHideTab) asm volatile("" : "+s"(syj), "+s"(cyj));
+      const double p0 = t.fx * cur[r][0], p1 = t.fx * cur[r][1];
+      const double w = from_west0(p1), e = from_east0(p0);
+      double f0 = t.mdiag * cur[r][0], f1 = t.mdiag * cur[r][1];
+      f0 = f0 + w;
+      f1 = f1 + p0;
+      f0 = f0 + p1;
+      f1 = f1 + e;
+      f0 = f0 + s0;
+      f1 = f1 + s1;
+      f0 = f0 + n0;
+      f1 = f1 + n1;
+      if (!COMB) {
+        f0 = 0.0 + f0;
+        f1 = 0.0 + f1;
+      }
+      if (MMS) {
+        f0 = f0 + forcing(T1, T2, t.sx0, t.cx0, syj, cyj);
+        f1 = f1 + forcing(T1, T2, t.sx1, t.cx1, syj, cyj);
+      }
+      if (COMB) {
+        f0 = lc5(c, f0, prev[r][0], yn[r][0], cur[r][0], fn[r][0]);
+        f1 = lc5(c, f1, prev[r][1], yn[r][1], cur[r][1], fn[r][1]);
+      }
+      if (MASK) {
+        f0 = t.in0 ? f0 : 0.0;
+        f1 = t.in1 ? f1 : 0.0;
+      }
+      prev[r][0] = f0;
+      prev[r][1] = f1;
+    }
+    s0 = m0;
+    s1 = m1;
+    m0 = n0;
+    m1 = n1;
   }
 }
 
@@ -120,11 +170,14 @@ struct TileGeo {
   int y0;          // row offset of a tile's first row from its first owned one
 };
 
-// the pass on one tile: K stages with the coefficients sc[8*m .. 8*m+6]
-template <int R, bool PER, bool MMS>
+// the pass on one tile: K stages with the coefficients sc[8*m .. 8*m+6].  CC:
+// constant coefficients, as the manufactured problem (not PER) always has
+template <int R, bool PER, bool CC>
 __device__ __forceinline__ void tile_pass(const TileGeo& g, const TileIO& o, ccdouble* sc, int strip, int rb,
                                           double2* lds, int nw)
 {
+  static_assert(PER || CC, "the manufactured problem has constant coefficients");
+  constexpr bool MMS = !PER;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
   const int64_t nx = g.nx, ny = g.ny;
@@ -141,18 +194,24 @@ __device__ __forceinline__ void tile_pass(const TileGeo& g, const TileIO& o, ccd
   }
   t.in0 = PER || (c0 >= 0 && c0 < nx);
   t.in1 = PER || (c1 >= 0 && c1 < nx);
+  t.fx = t.fy = t.mdiag = 0.0;
+  if (CC) {
+    t.fx = ((ccdouble*)g.fx)[0];
+    t.fy = ((ccdouble*)g.fy)[0];
+    t.mdiag = -((t.fx + t.fx) + (t.fy + t.fy));
+  }
   t.Dw0 = t.De0 = t.Dw1 = t.De1 = t.sx0 = t.sx1 = t.cx0 = t.cx1 = 0.0;
   if (t.in0) {
-    t.Dw0 = g.fx[c0];
-    t.De0 = g.fx[c0 + 1];
+    if (!CC) t.Dw0 = g.fx[c0];
+    if (!CC) t.De0 = g.fx[c0 + 1];
     if (MMS) {
       t.sx0 = g.sx[c0];
       t.cx0 = g.cx[c0];
     }
   }
   if (t.in1) {
-    t.Dw1 = g.fx[c1];
-    t.De1 = g.fx[c1 + 1];
+    if (!CC) t.Dw1 = g.fx[c1];
+    if (!CC) t.De1 = g.fx[c1 + 1];
     if (MMS) {
       t.sx1 = g.sx[c1];
       t.cx1 = g.cx[c1];
@@ -170,8 +229,8 @@ __device__ __forceinline__ void tile_pass(const TileGeo& g, const TileIO& o, ccd
     }
     jr[r] = j;
     const bool ok = PER || (j >= 0 && j < ny);
-    t.Ds[r] = ok ? fy[j] : 0.0;
-    t.Dn[r] = ok ? fy[j + 1] : 0.0;
+    t.Ds[r] = (ok && !CC) ? fy[j] : 0.0;
+    t.Dn[r] = (ok && !CC) ? fy[j + 1] : 0.0;
     t.sy[r] = (MMS && ok) ? sy[j] : 0.0;
     t.cy[r] = (MMS && ok) ? cy[j] : 0.0;
   }
@@ -248,8 +307,9 @@ __device__ __forceinline__ void tile_pass(const TileGeo& g, const TileIO& o, ccd
     __syncthreads();
     if (needed(m + 1)) {
       const double2 S = south(m & 1), N = north(m & 1);
-      if (!PER && mask) tile_stage<R, MMS, true, true>(t, ny, cf, prev, cur, yn, fn, S, N);
-      else tile_stage<R, MMS, false, true>(t, ny, cf, prev, cur, yn, fn, S, N);
+      if (CC && !PER && mask) tile_stage_cc<R, MMS, true, true>(t, ny, cf, prev, cur, yn, fn, S, N);
+      else if (CC) tile_stage_cc<R, MMS, false, true>(t, ny, cf, prev, cur, yn, fn, S, N);
+      else tile_stage<R, true>(t, cf, prev, cur, yn, fn, S, N);
       publish((m + 1) & 1, prev);
     }
   };
@@ -293,13 +353,14 @@ __device__ __forceinline__ void tile_pass(const TileGeo& g, const TileIO& o, ccd
     __syncthreads();
     if (needed(L)) {
       const double2 S = south(o.K & 1), N = north(o.K & 1);
-      tile_stage<R, MMS, false, false>(t, ny, cf, A, B, yn, fn, S, N);
+      if (CC) tile_stage_cc<R, MMS, false, false>(t, ny, cf, A, B, yn, fn, S, N);
+      else tile_stage<R, false>(t, cf, A, B, yn, fn, S, N);
       st(o.outF, A);
     }
   }
 }
 
-template <int R, bool PER, bool MMS>
+template <int R, bool PER, bool CC>
 __global__ __launch_bounds__(kTileThreads) void k_tile(const TileGeo g, const TileOps o)
 {
   extern __shared__ double2 tile_lds[];
@@ -309,7 +370,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile(const TileGeo g, const Ti
   const unsigned q = nb >> 3, r = nb & 7u, xcd = b & 7u, loc = b >> 3;
   const unsigned tile = xcd * q + (xcd < r ? xcd : r) + loc;
   const int strip = (int)(tile % (unsigned)g.strips), rb = (int)(tile / (unsigned)g.strips);
-  tile_pass<R, PER, MMS>(g, o, (ccdouble*)o.c, strip, rb, tile_lds, (int)(blockDim.x / kWave));
+  tile_pass<R, PER, CC>(g, o, (ccdouble*)o.c, strip, rb, tile_lds, (int)(blockDim.x / kWave));
 }
 
 // column strips and owned rows of tiles of `rows` rows with halo H.  A
@@ -376,7 +437,8 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_batch(const TileSlot* __r
   o.outB = t.buf[2 * par + 1];
   o.outF = t.buf[2 * par];
   ccdouble* sc = (ccdouble*)(t.coef + 8 * (j - 2));
-  if (t.per) tile_pass<R, true, false>(g, o, sc, ref.strip, ref.rb, tile_lds, kTileBatchWaves);
+  if (t.per && t.cc) tile_pass<R, true, true>(g, o, sc, ref.strip, ref.rb, tile_lds, kTileBatchWaves);
+  else if (t.per) tile_pass<R, true, false>(g, o, sc, ref.strip, ref.rb, tile_lds, kTileBatchWaves);
   else tile_pass<R, false, true>(g, o, sc, ref.strip, ref.rb, tile_lds, kTileBatchWaves);
 }
 
@@ -416,9 +478,10 @@ void launch_tile(DiffusionProblem* P, const TileCfg& t, const TileOps& o, hipStr
   const unsigned nt = (unsigned)(t.nw * kWave);
   const size_t lds = sizeof(double2) * 2 * 2 * kWave * (size_t)t.nw;  // at most 64 KiB
   const bool per = P->p.kind == DIFFUSION_CEDA_PERIODIC;
-#define CEDA_TILE(RR)                                                                             \
-  if (per) hipLaunchKernelGGL((k_tile<RR, true, false>), dim3(grid), dim3(nt), lds, s, g, o);     \
-  else hipLaunchKernelGGL((k_tile<RR, false, true>), dim3(grid), dim3(nt), lds, s, g, o);
+#define CEDA_TILE(RR)                                                                                      \
+  if (!per) hipLaunchKernelGGL((k_tile<RR, false, true>), dim3(grid), dim3(nt), lds, s, g, o);              \
+  else if (P->constant_faces) hipLaunchKernelGGL((k_tile<RR, true, true>), dim3(grid), dim3(nt), lds, s, g, o); \
+  else hipLaunchKernelGGL((k_tile<RR, true, false>), dim3(grid), dim3(nt), lds, s, g, o);
   switch (t.R) {
     case 1: CEDA_TILE(1) break;
     case 2: CEDA_TILE(2) break;
