@@ -9,8 +9,11 @@
 // oracle's serial loops.  Reductions are two-pass and deterministic: a fixed
 // grid reduces each lane's strided elements in index order, then wave64
 // butterflies (__shfl_xor), then LDS across the 4 wavefronts of a workgroup,
-// then one workgroup combines the per-group partials in fixed order.
+// then one workgroup combines the per-group partials in fixed order and stores
+// the results to host memory.
+#include <atomic>
 #include <cfloat>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 
@@ -230,39 +233,79 @@ __global__ __launch_bounds__(kBlock) void k_reduce(int64_t n, int nacc, R r, dou
   }
 }
 
-template <int K>
-__global__ __launch_bounds__(kBlock) void k_reduce_final(int nblocks, int nacc,
-                                                         const double* partials, double* out)
+// Workgroup x combines the partials of accumulators x*NACC .. x*NACC + NACC-1,
+// all of them at once, and stores the results to host memory.
+template <int K, int NACC>
+__global__ __launch_bounds__(kBlock) void k_reduce_final(int nblocks, int nacc, const double* partials, double* out)
 {
-  __shared__ double s[kBlock / kWave];
+  __shared__ double s[kBlock / kWave][NACC];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  for (int k = 0; k < nacc; k++) {
-    double v = rinit<K>();
-    for (int b = threadIdx.x; b < nblocks; b += kBlock) v = rcombine<K>(v, partials[(int64_t)b * nacc + k]);
-    v = wave_reduce<K>(v);
-    if (lane == 0) s[wave] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double t = s[0];
-      for (int w = 1; w < kBlock / kWave; w++) t = rcombine<K>(t, s[w]);
-      out[k] = t;
+  const int base = blockIdx.x * NACC, na = nacc - base < NACC ? nacc - base : NACC;
+  double v[NACC];
+#pragma unroll
+  for (int k = 0; k < NACC; k++) v[k] = rinit<K>();
+  for (int b = threadIdx.x; b < nblocks; b += kBlock) {
+#pragma unroll
+    for (int k = 0; k < NACC; k++) {
+      if (k >= na) break;
+      v[k] = rcombine<K>(v[k], partials[(int64_t)b * nacc + base + k]);
     }
-    __syncthreads();
   }
+#pragma unroll
+  for (int k = 0; k < NACC; k++) {
+    if (k >= na) break;
+    const double t = wave_reduce<K>(v[k]);
+    if (lane == 0) s[wave][k] = t;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < na) {
+    double t = s[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < kBlock / kWave; w++) t = rcombine<K>(t, s[w][threadIdx.x]);
+    __hip_atomic_store(out + base + threadIdx.x, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// The host waits for the results themselves: it marks every slot that a launch
+// will store to with a NaN that no operation produces and reads until all are
+// overwritten.  A result that is this very NaN, or a longer wait than kSpin, is
+// left to the stream.  The stream is in order, so with the results everything
+// issued before them is done too.  A dot product of up to 131072 entries:
+// 18.4 us with a copy of the result and a wait for the stream, 16.2 with the
+// result stored by the kernel, 10.9 with this wait.  (The last of the first
+// kernel's workgroups doing the second's work was measured: 15.1 us for up to
+// 32 workgroups, but 19 for 256 and 51 for 2048, for the fences.)
+constexpr uint64_t kPending = 0xfff8dead5eedc0deull;
+constexpr std::chrono::microseconds kSpin(500);
+void mark_results(Exec* ex, int nacc)
+{
+  volatile uint64_t* r = reinterpret_cast<volatile uint64_t*>(ex->h_result);
+  for (int k = 0; k < nacc; k++) r[k] = kPending;
+  std::atomic_thread_fence(std::memory_order_release);
+}
+void wait_results(Exec* ex, int nacc)
+{
+  const volatile uint64_t* r = reinterpret_cast<const volatile uint64_t*>(ex->h_result);
+  const auto until = std::chrono::steady_clock::now() + kSpin;
+  int k = 0;
+  do {
+    for (int spin = 0; spin < 256 && k < nacc; spin++)
+      while (k < nacc && r[k] != kPending) k++;
+  } while (k < nacc && std::chrono::steady_clock::now() < until);
+  std::atomic_thread_fence(std::memory_order_acquire);
+  if (k < nacc) CEDA_HIP_CHECK(hipStreamSynchronize(ex->stream));
 }
 
 template <int K, int NACC, class R>
 const double* run_reduce(Exec* ex, int64_t n, int nacc, const R& r)
 {
   const unsigned g = reduce_grid(n);
+  mark_results(ex, nacc);
   hipLaunchKernelGGL((k_reduce<K, NACC, R>), dim3(g), dim3(kBlock), 0, ex->stream, n, nacc, r, ex->d_partials);
+  hipLaunchKernelGGL((k_reduce_final<K, NACC>), dim3(1), dim3(kBlock), 0, ex->stream, (int)g, nacc, ex->d_partials,
+                     ex->h_result);
   CEDA_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(k_reduce_final<K>, dim3(1), dim3(kBlock), 0, ex->stream, (int)g, nacc,
-                     ex->d_partials, ex->d_result);
-  CEDA_HIP_CHECK(hipGetLastError());
-  CEDA_HIP_CHECK(hipMemcpyAsync(ex->h_result, ex->d_result, sizeof(double) * nacc,
-                                hipMemcpyDeviceToHost, ex->stream));
-  CEDA_HIP_CHECK(hipStreamSynchronize(ex->stream));
+  wait_results(ex, nacc);
   return ex->h_result;
 }
 
@@ -595,8 +638,7 @@ struct DotGroups {
   const double* y[NVHIP_MAX_FUSED];
   int nv;
 };
-__global__ __launch_bounds__(kBlock) void k_dotmulti_groups(int64_t n, DotGroups r,
-                                                            double* partials)
+__global__ __launch_bounds__(kBlock) void k_dotmulti_groups(int64_t n, DotGroups r, double* partials)
 {
   const int base = blockIdx.y * 8, ntot = 8 * gridDim.y;
   double acc[8];
@@ -643,14 +685,12 @@ static void dotmulti_groups(int nvec, N_Vector x, N_Vector* Y, sunrealtype* d)
   const int64_t n = vlen(x);
   const unsigned g = reduce_grid(n);
   const int ngroups = (nvec + 7) / 8;
+  mark_results(ex, 8 * ngroups);
   hipLaunchKernelGGL(k_dotmulti_groups, dim3(g, ngroups), dim3(kBlock), 0, ex->stream, n, r, ex->d_partials);
+  hipLaunchKernelGGL((k_reduce_final<RSUM, 8>), dim3(ngroups), dim3(kBlock), 0, ex->stream, (int)g, 8 * ngroups,
+                     ex->d_partials, ex->h_result);
   CEDA_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(k_reduce_final<RSUM>, dim3(1), dim3(kBlock), 0, ex->stream, (int)g, 8 * ngroups,
-                     ex->d_partials, ex->d_result);
-  CEDA_HIP_CHECK(hipGetLastError());
-  CEDA_HIP_CHECK(hipMemcpyAsync(ex->h_result, ex->d_result, sizeof(double) * nvec, hipMemcpyDeviceToHost,
-                                ex->stream));
-  CEDA_HIP_CHECK(hipStreamSynchronize(ex->stream));
+  wait_results(ex, 8 * ngroups);
   for (int k = 0; k < nvec; k++) d[k] = ex->h_result[k];
 }
 

@@ -88,8 +88,7 @@ constexpr int kMaxAcc = 64;          // accumulators per reduction (DotProdMulti
 struct Exec {
   hipStream_t stream = nullptr;
   double* d_partials = nullptr;      // kMaxReduceBlocks * kMaxAcc
-  double* d_result = nullptr;        // kMaxAcc
-  double* h_result = nullptr;        // pinned, kMaxAcc
+  double* h_result = nullptr;        // pinned, kMaxAcc; reductions store to it
   int num_cu = 256;
 };
 

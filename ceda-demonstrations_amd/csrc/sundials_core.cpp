@@ -38,7 +38,6 @@ SUNErrCode SUNContext_Create(SUNComm, SUNContext* ctx)
   }
   CEDA_HIP_CHECK(ceda::dev_malloc(&c->exec.d_partials,
                            sizeof(double) * ceda::kMaxReduceBlocks * ceda::kMaxAcc));
-  CEDA_HIP_CHECK(ceda::dev_malloc(&c->exec.d_result, sizeof(double) * ceda::kMaxAcc));
   CEDA_HIP_CHECK(ceda::host_malloc(&c->exec.h_result, sizeof(double) * ceda::kMaxAcc,
                                hipHostMallocDefault));
   int dev = 0;
@@ -56,7 +55,6 @@ SUNErrCode SUNContext_Free(SUNContext* ctx)
   SUNContext c = *ctx;
   CEDA_HIP_CHECK(hipStreamSynchronize(c->exec.stream));
   CEDA_HIP_CHECK(ceda::dev_free(c->exec.d_partials));
-  CEDA_HIP_CHECK(ceda::dev_free(c->exec.d_result));
   CEDA_HIP_CHECK(ceda::host_free(c->exec.h_result));
   {
     std::lock_guard<std::recursive_mutex> g(ceda::device_sync_mutex());
