@@ -510,6 +510,22 @@ void DiffusionParams_Default(DiffusionParams* p, int kind)
   }
 }
 
+// Rows per wavefront of k_stencil until a problem is tuned: the most that leave
+// 1024 workgroups, four per CU.  A wavefront's rows follow one another, a
+// memory latency each, so small grids want one row (RHS at 640 x 500: 3.1 us
+// with 1, 5.2 with 8; 64^2: 2.3, 4.8), while large ones re-read less with more
+// (2048^2 Dirichlet: 17.3 us with 1, 14.1 with 8; 1024^2: 6.3 with 1, 5.8 with
+// 2, 6.9 with 8).  The stage kernel streams three more vectors and gains
+// nothing beyond 2 (1024^2: 8.2 us with 1, 7.6 with 2, 10.2 with 8).
+static int default_rows(int64_t nx, int64_t ny, int most)
+{
+  const int64_t cols = kWave * (nx % 2 == 0 ? 2 : 1);
+  const int64_t groups = (nx + cols - 1) / cols * ((ny + 3) / 4);
+  int rows = 1;
+  while (rows < most && groups >= 2048 * rows) rows *= 2;
+  return rows;
+}
+
 DiffusionProblem* DiffusionProblem_Create(const DiffusionParams* prm, SUNContext ctx)
 {
   if (!prm || !ctx) return nullptr;
@@ -580,8 +596,8 @@ DiffusionProblem* DiffusionProblem_Create(const DiffusionParams* prm, SUNContext
   upload_tables(P);
   P->diag = N_VNew_HipNative(P->n, ctx);
   N_VConst(1.0, P->diag);
-  P->cfg[0] = StencilCfg{0, 8, 0};
-  P->cfg[1] = StencilCfg{0, 2, 0};
+  P->cfg[0] = StencilCfg{0, default_rows(nx, ny, 8), 0};
+  P->cfg[1] = StencilCfg{0, default_rows(nx, ny, 2), 0};
   P->cfg[2] = StencilCfg{0, 32, 0};
   return P;
 }
