@@ -407,10 +407,9 @@ void run_marching(DiffusionBatch* B, const std::vector<int>& planned, bool adapt
 // kTileCells cells, each to its end before the next: the six vectors of a
 // sub-batch then stay in the 256 MB last-level cache over its passes, its
 // problems need about the same number of passes, and the host prepares the
-// next one meanwhile.  256 uneven problems to t = 0.06: a call 741 -> 593 ms
-// (312 of them the passes, 300 creation and release of the problems), 24 ragged
-// ones to t = 0.01: 112 -> 30 ms, where the marching tiles also timed seven
-// tile heights for every size class.
+// next one meanwhile.  The step groups of 256 uneven problems to t = 0.06 take 290 ms;
+// 24 ragged ones to t = 0.01 14 ms, a whole call 112 -> 20 ms, where the marching
+// tiles also timed seven tile heights for every size class.
 constexpr int64_t kTileCells = (int64_t)4 << 20;
 // below this many tiles of 64 rows a pass runs on tiles of 32 rows (own 10
 // rows instead of 42, half the time per tile): the GPU has 256 CUs
@@ -582,6 +581,7 @@ DiffusionBatch* DiffusionBatch_Create(int nprob, const DiffusionParams* params,
   B->ex = ceda::context_exec(ctx);
   B->method = (method == ARKODE_LSRK_RKL_2) ? M_RKL : M_RKC;
   B->probs.resize(nprob);
+  ceda::SlabScope slabs;  // the problems' vectors and tables
   for (int k = 0; k < nprob; k++) {
     BProb& b = B->probs[k];
     b.P = DiffusionProblem_Create(&params[k], ctx);

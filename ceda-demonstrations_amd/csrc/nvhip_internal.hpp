@@ -31,17 +31,32 @@ namespace ceda {
 // every such call hold this lock, so that integrators on separate contexts
 // can be driven from separate host threads.
 std::recursive_mutex& device_sync_mutex();
+// Device memory of many objects made together (a batch's problems): while a
+// SlabScope lives, its thread's dev_malloc takes pieces of shared slabs.  A
+// piece is not used twice; a slab is freed with its last piece once its scope
+// has ended.  The vectors and tables of 256 problems are 2,560 pieces: freeing
+// each took 225 ms (hipFree waits for the device), their 14 slabs take 4; making
+// them went from 37 to 10 ms.
+class SlabScope {
+ public:
+  SlabScope();
+  ~SlabScope();
+  SlabScope(const SlabScope&) = delete;
+  SlabScope& operator=(const SlabScope&) = delete;
+
+ private:
+  friend hipError_t dev_malloc_bytes(void** p, size_t bytes);
+  SlabScope* outer_;
+  char* slab_ = nullptr;  // the slab in use
+  size_t used_ = 0, size_ = 0, total_ = 0;
+};
+hipError_t dev_malloc_bytes(void** p, size_t bytes);
 template <class T>
 inline hipError_t dev_malloc(T** p, size_t bytes)
 {
-  std::lock_guard<std::recursive_mutex> g(device_sync_mutex());
-  return hipMalloc(p, bytes);
+  return dev_malloc_bytes(reinterpret_cast<void**>(p), bytes);
 }
-inline hipError_t dev_free(void* p)
-{
-  std::lock_guard<std::recursive_mutex> g(device_sync_mutex());
-  return hipFree(p);
-}
+hipError_t dev_free(void* p);
 template <class T>
 inline hipError_t host_malloc(T** p, size_t bytes, unsigned flags)
 {

@@ -8,8 +8,10 @@
 // reduction workspace (device partials + pinned host result).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 
 #include "nvhip_internal.hpp"
 
@@ -23,6 +25,84 @@ std::recursive_mutex& device_sync_mutex()
 {
   static std::recursive_mutex mu;
   return mu;
+}
+
+namespace {
+struct Slab {
+  size_t size;
+  int live;   // pieces not yet freed
+  bool open;  // its scope may still take pieces
+};
+// by address, under device_sync_mutex; never destroyed: objects of static
+// lifetime may be released after it would be
+std::map<char*, Slab>& slabs()
+{
+  static auto* m = new std::map<char*, Slab>();
+  return *m;
+}
+thread_local SlabScope* t_slab = nullptr;
+// slabs double from 4 MB to 256 MB; larger pieces than 16 MB are allocated by
+// themselves (a fixed cost per call matters little there)
+constexpr size_t kSlabMin = (size_t)4 << 20, kSlabMax = (size_t)256 << 20, kPieceMax = (size_t)16 << 20;
+
+hipError_t slab_close(char* p)
+{
+  auto it = slabs().find(p);
+  it->second.open = false;
+  if (it->second.live > 0) return hipSuccess;
+  slabs().erase(it);
+  return hipFree(p);
+}
+}  // namespace
+
+SlabScope::SlabScope() : outer_(t_slab) { t_slab = this; }
+SlabScope::~SlabScope()
+{
+  t_slab = outer_;
+  std::lock_guard<std::recursive_mutex> g(device_sync_mutex());
+  if (slab_) CEDA_HIP_CHECK(slab_close(slab_));
+}
+
+hipError_t dev_malloc_bytes(void** p, size_t bytes)
+{
+  std::lock_guard<std::recursive_mutex> g(device_sync_mutex());
+  SlabScope* S = t_slab;
+  if (!S || bytes == 0 || bytes > kPieceMax) return hipMalloc(p, bytes);
+  const size_t piece = (bytes + 255) / 256 * 256;
+  if (S->used_ + piece > S->size_) {
+    const size_t want = std::max(piece, std::min(kSlabMax, std::max(kSlabMin, S->total_)));
+    void* q = nullptr;
+    if (hipMalloc(&q, want) != hipSuccess) {  // no room for a slab: perhaps for the piece
+      (void)hipGetLastError();
+      return hipMalloc(p, bytes);
+    }
+    if (S->slab_) CEDA_HIP_CHECK(slab_close(S->slab_));
+    S->slab_ = static_cast<char*>(q);
+    S->used_ = 0;
+    S->size_ = want;
+    S->total_ += want;
+    slabs()[S->slab_] = Slab{want, 0, true};
+  }
+  *p = S->slab_ + S->used_;
+  S->used_ += piece;
+  slabs()[S->slab_].live++;
+  return hipSuccess;
+}
+
+hipError_t dev_free(void* p)
+{
+  std::lock_guard<std::recursive_mutex> g(device_sync_mutex());
+  auto it = slabs().upper_bound(static_cast<char*>(p));
+  if (p && it != slabs().begin()) {
+    --it;
+    if (static_cast<char*>(p) < it->first + it->second.size) {
+      if (--it->second.live > 0 || it->second.open) return hipSuccess;
+      char* base = it->first;
+      slabs().erase(it);
+      return hipFree(base);
+    }
+  }
+  return hipFree(p);
 }
 }  // namespace ceda
 
