@@ -1516,20 +1516,24 @@ __global__ __launch_bounds__(kBlock) void k_cg_iter(int n, double rx, double ry,
 // One workgroup iterates one pair until it converges (or for `iters`
 // iterations), with r in registers throughout.  Up to kCgLdsSide^2 cells x and
 // Ap are in registers too and p in LDS: an iteration touches no memory, and is
-// bound by its three barriers' phases.  Above, p and x stay in memory: each
-// iteration reads and writes p and x once and reads p's five points twice (48
-// bytes per cell instead of 64), and the pairs being solved, one per CU, stay
-// in the 256 MB of last-level cache (2 x 75 MB at 192^2) where k_cg_iter, which
-// advances every pair by one iteration per launch, streams them all from HBM.
+// bound by its three barriers' phases.  Above, x and the p that the LDS does not
+// hold stay in memory: an iteration reads and writes x once, and of that p reads
+// and writes the cells once and their five points twice (16 and 32 bytes per
+// cell); the pairs being solved, one per CU, stay in the 256 MB of last-level
+// cache, where k_cg_iter, which advances every pair by one iteration per launch,
+// streams them all from HBM (64 bytes).
 // Cells are units of W (pairs with 16-byte accesses for even n): unit m of a
-// thread is unit m T + tid of the grid.
-// 1,024 pairs, time per iteration: 192^2 257 us, 7.1 TB/s of cache (537 us,
-// 4.5 TB/s, by k_cg_iter), 128^2 45 us (223), 100^2 33 us (140), 64^2 17 us (48);
-// 1,024 pairs of 192^2 to 1e-12 with 490 iterations 178 ms (380).
+// thread is unit m T + tid of the grid, and the first CPL / W units of every
+// thread are in LDS, so that the place of a unit and, but for the units at the
+// border, of its neighbours is known when the loops are unrolled.
+// 1,024 pairs, time per iteration: 192^2 156 us, bound by 32 bytes per cell of
+// cache (257 us, 7.1 TB/s, with all p in memory; 537 us by k_cg_iter), 160^2
+// 87 us, 128^2 32 us (223 by k_cg_iter), 100^2 26 us (140).
 constexpr int kCgLdsSide = 128;   // p in LDS: 128 KiB
 constexpr int kCgRegSide = 192;   // r in registers: 36 cells per thread
 constexpr int kCgCellsLds = 16;   // cells per thread, p in LDS
-constexpr int kCgCellsMem = 36;   // cells per thread, p in memory
+constexpr int kCgCellsMem = 36;   // cells per thread, p partly in memory
+constexpr int kCgCellsHalf = 18;  // of them in LDS: 144 KiB
 
 __device__ inline double cg_wave_sum(double v)  // the wavefront's sum, in every lane
 {
@@ -1552,14 +1556,17 @@ __device__ inline double cg_block_sum(double v, double* sh)
   return t;
 }
 
-template <int T, int CPT, int W, bool LDS>
+template <int T, int CPT, int CPL, int W>
 __global__ __launch_bounds__(T) void k_cg_solve(int n, double rx, double ry, double idg, double tol2, int iters,
                                                 double* __restrict__ x, double* __restrict__ r,
                                                 double* __restrict__ p, CGState* __restrict__ st)
 {
-  constexpr int M = CPT / W;  // units per thread
+  constexpr int M = CPT / W;   // units per thread
+  constexpr int ML = CPL / W;  // of them, the first ones' p is in LDS
+  constexpr bool LDS = CPL == CPT;
+  constexpr int kl = ML * T * W;
   constexpr int kFlight = 3;
-  extern __shared__ double pl[];
+  extern __shared__ __attribute__((aligned(16))) double pl[];
   __shared__ double sh[2][T / kWave];
   CGState S = st[blockIdx.x];
   if (S.done) return;
@@ -1568,24 +1575,32 @@ __global__ __launch_bounds__(T) void k_cg_solve(int n, double rx, double ry, dou
   double* __restrict__ rs = r + o;
   double* ps = p + o;
   const int h = n / W, nu = h * n, di = T % h, dj = T / h, i0 = (int)threadIdx.x % h, j0 = (int)threadIdx.x / h;
-  auto pld = [&](int k, double (&v)[W]) {
-    if (LDS) {
-#pragma unroll
-      for (int t = 0; t < W; t++) v[t] = pl[k + t];
+  // p: cells below kl in LDS, the others in memory.  side: 1 (LDS) or 0 for an
+  // access whose unit tells, 2 where a unit's neighbours may lie on either side
+  auto pld = [&](int side, int k, double (&v)[W]) {
+    if (side == 1 || (side == 2 && k < kl)) {
+      if (W == 2) {
+        const double2 u = *reinterpret_cast<const double2*>(pl + k);
+        v[0] = u.x;
+        v[W - 1] = u.y;
+      } else v[0] = pl[k];
     } else if (W == 2) {
       const double2 u = *reinterpret_cast<const double2*>(ps + k);
       v[0] = u.x;
       v[W - 1] = u.y;
     } else v[0] = ps[k];
   };
-  auto p1 = [&](int k) { return LDS ? pl[k] : ps[k]; };
-  auto pst = [&](int k, const double (&v)[W]) {
-    if (LDS) {
-#pragma unroll
-      for (int t = 0; t < W; t++) pl[k + t] = v[t];
-    } else if (W == 2) *reinterpret_cast<double2*>(ps + k) = make_double2(v[0], v[W - 1]);
-    else ps[k] = v[0];
+  auto p1 = [&](int side, int k) { return (side == 1 || (side == 2 && k < kl)) ? pl[k] : ps[k]; };
+  auto pst = [&](int side, int k, const double (&v)[W]) {
+    double* q = side == 1 ? pl : ps;
+    if (W == 2) *reinterpret_cast<double2*>(q + k) = make_double2(v[0], v[W - 1]);
+    else q[k] = v[0];
   };
+  // where unit m's cells, and those a row (at most T * W cells) before and
+  // after them, lie
+  auto own = [](int m) { return m < ML ? 1 : 0; };
+  auto below = [](int m) { return m < ML ? 1 : (m == ML ? 2 : 0); };
+  auto above = [](int m) { return m < ML - 1 || ML == M ? 1 : (m == ML - 1 ? 2 : 0); };
   // f(m, unit, column unit, row) over the thread's units
   auto each = [&](auto&& f) {
     int i = i0, j = j0, q0 = (int)threadIdx.x;
@@ -1604,15 +1619,15 @@ __global__ __launch_bounds__(T) void k_cg_solve(int n, double rx, double ry, dou
     }
   };
   // (I - rx Dxx - ry Dyy) p at a unit
-  auto apply = [&](int q, int i, int j, double (&c)[W], double (&v)[W]) {
+  auto apply = [&](int m, int q, int i, int j, double (&c)[W], double (&v)[W]) {
     const int k = q * W, ic = i * W;
     double s[W], no[W];
-    pld(k, c);
-    const double w = ic > 0 ? p1(k - 1) : 0.0, e = ic + W < n ? p1(k + W) : 0.0;
+    pld(own(m), k, c);
+    const double w = ic > 0 ? p1(below(m), k - 1) : 0.0, e = ic + W < n ? p1(above(m), k + W) : 0.0;
 #pragma unroll
     for (int t = 0; t < W; t++) s[t] = no[t] = 0.0;
-    if (j > 0) pld(k - n, s);
-    if (j < n - 1) pld(k + n, no);
+    if (j > 0) pld(below(m), k - n, s);
+    if (j < n - 1) pld(above(m), k + n, no);
 #pragma unroll
     for (int t = 0; t < W; t++)
       v[t] = op5(c[t], t > 0 ? c[t > 0 ? t - 1 : 0] : w, t < W - 1 ? c[t < W - 1 ? t + 1 : 0] : e, s[t], no[t], rx, ry);
@@ -1622,10 +1637,8 @@ __global__ __launch_bounds__(T) void k_cg_solve(int n, double rx, double ry, dou
 #pragma unroll
     for (int t = 0; t < W; t++) {
       rr[m][t] = rs[q * W + t];
-      if (LDS) {
-        xr[LDS ? m : 0][t] = xs[q * W + t];
-        pl[q * W + t] = ps[q * W + t];
-      }
+      if (LDS) xr[LDS ? m : 0][t] = xs[q * W + t];
+      if (m < ML) pl[q * W + t] = ps[q * W + t];
     }
   });
   const int last = S.iters + iters;
@@ -1634,16 +1647,16 @@ __global__ __launch_bounds__(T) void k_cg_solve(int n, double rx, double ry, dou
     // read p with the sum that ended it)
     each([&](int m, int q, int, int) {
       double v[W];
-      pld(q * W, v);
+      pld(own(m), q * W, v);
 #pragma unroll
       for (int t = 0; t < W; t++) v[t] = rr[m][t] * idg + S.beta * v[t];
-      pst(q * W, v);
+      pst(own(m), q * W, v);
     });
     __syncthreads();
     double pap = 0.0;
     each([&](int m, int q, int i, int j) {
       double c[W], v[W];
-      apply(q, i, j, c, v);
+      apply(m, q, i, j, c, v);
 #pragma unroll
       for (int t = 0; t < W; t++) {
         pap += c[t] * v[t];
@@ -1655,14 +1668,14 @@ __global__ __launch_bounds__(T) void k_cg_solve(int n, double rx, double ry, dou
     each([&](int m, int q, int i, int j) {
       double c[W], v[W];
       if (LDS) {
-        pld(q * W, c);
+        pld(1, q * W, c);
 #pragma unroll
         for (int t = 0; t < W; t++) {
           v[t] = ap[LDS ? m : 0][t];
           xr[LDS ? m : 0][t] += alpha * c[t];
         }
       } else {
-        apply(q, i, j, c, v);
+        apply(m, q, i, j, c, v);
         if (W == 2) {
           double2* xp = reinterpret_cast<double2*>(xs + q * W);
           const double2 xv = *xp;
@@ -1686,10 +1699,8 @@ __global__ __launch_bounds__(T) void k_cg_solve(int n, double rx, double ry, dou
 #pragma unroll
     for (int t = 0; t < W; t++) {
       rs[q * W + t] = rr[m][t];
-      if (LDS) {
-        xs[q * W + t] = xr[LDS ? m : 0][t];
-        ps[q * W + t] = pl[q * W + t];
-      }
+      if (LDS) xs[q * W + t] = xr[LDS ? m : 0][t];
+      if (m < ML) ps[q * W + t] = pl[q * W + t];
     }
   });
   if (threadIdx.x == 0) st[blockIdx.x] = S;
@@ -2282,32 +2293,32 @@ void adam_step(LearnedPrec* L, double lr)
 
 // up to `iters` Jacobi-PCG iterations of every pair on one CU each; false
 // where the sides are too large for it (or the LDS is refused)
-template <int T, int CPT, int W, bool LDS>
+template <int T, int CPT, int CPL, int W>
 bool launch_cg_solve(int nsamp, int n, double rx, double ry, double idg, double tol2, int iters, double* x, double* r,
                      double* p, CGState* st, hipStream_t s)
 {
-  const size_t lds = LDS ? sizeof(double) * (size_t)n * n : 0;
+  const size_t lds = sizeof(double) * (size_t)std::min(n * n, T * CPL);
   if (lds > 32768) {
     static const hipError_t allowed = hipFuncSetAttribute(
-        (const void*)k_cg_solve<T, CPT, W, LDS>, hipFuncAttributeMaxDynamicSharedMemorySize, 8 * T * CPT);
+        (const void*)k_cg_solve<T, CPT, CPL, W>, hipFuncAttributeMaxDynamicSharedMemorySize, 8 * T * CPL);
     if (allowed != hipSuccess) {
       (void)hipGetLastError();
       return false;
     }
   }
-  hipLaunchKernelGGL((k_cg_solve<T, CPT, W, LDS>), dim3(nsamp), dim3(T), lds, s, n, rx, ry, idg, tol2, iters, x, r, p, st);
+  hipLaunchKernelGGL((k_cg_solve<T, CPT, CPL, W>), dim3(nsamp), dim3(T), lds, s, n, rx, ry, idg, tol2, iters, x, r, p, st);
   return true;
 }
 bool cg_solve(int nsamp, int n, double rx, double ry, double idg, double tol2, int iters, double* x, double* r,
               double* p, CGState* st, hipStream_t s)
 {
-#define CEDA_CG(T, C, L)                                                                                       \
-  return n % 2 == 0 ? launch_cg_solve<T, C, 2, L>(nsamp, n, rx, ry, idg, tol2, iters, x, r, p, st, s)          \
-                    : launch_cg_solve<T, C, 1, L>(nsamp, n, rx, ry, idg, tol2, iters, x, r, p, st, s)
-  if (n * n <= 256 * kCgCellsLds) CEDA_CG(256, kCgCellsLds, true);
-  if (n * n <= 512 * kCgCellsLds) CEDA_CG(512, kCgCellsLds, true);
-  if (n <= kCgLdsSide) CEDA_CG(1024, kCgCellsLds, true);
-  if (n <= kCgRegSide) CEDA_CG(1024, kCgCellsMem, false);
+#define CEDA_CG(T, C, CL)                                                                                      \
+  return n % 2 == 0 ? launch_cg_solve<T, C, CL, 2>(nsamp, n, rx, ry, idg, tol2, iters, x, r, p, st, s)         \
+                    : launch_cg_solve<T, C, CL, 1>(nsamp, n, rx, ry, idg, tol2, iters, x, r, p, st, s)
+  if (n * n <= 256 * kCgCellsLds) CEDA_CG(256, kCgCellsLds, kCgCellsLds);
+  if (n * n <= 512 * kCgCellsLds) CEDA_CG(512, kCgCellsLds, kCgCellsLds);
+  if (n <= kCgLdsSide) CEDA_CG(1024, kCgCellsLds, kCgCellsLds);
+  if (n <= kCgRegSide) CEDA_CG(1024, kCgCellsMem, kCgCellsHalf);
 #undef CEDA_CG
   return false;
 }
