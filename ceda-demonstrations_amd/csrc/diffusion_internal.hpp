@@ -88,6 +88,7 @@ void launch_rhs_entry(DiffusionProblem* P, const StageEntry* e, hipStream_t s);
 // e[0].yjm1, e[0].yjm2, e[0].yn, e[0].fn; stage K-1 is written to e[K-2].out
 // and stage K to e[K-1].out (K = 1..4).  rows = output rows per wavefront
 // tile, nt = non-temporal streams.  Bitwise equal to K single-stage launches.
+int pass_fill_rows(const DiffusionProblem* P, int K, int nt, int rounds);
 void launch_pass(DiffusionProblem* P, int K, int rows, int nt, const StageEntry* e, hipStream_t s);
 // halo lanes of a K-stage pass (each side of a wavefront strip)
 int pass_halo_lanes(int K, int cpl);

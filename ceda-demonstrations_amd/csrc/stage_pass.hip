@@ -62,17 +62,17 @@ typedef __attribute__((address_space(1))) const d2v gcd2v;
 typedef __attribute__((address_space(1))) d2v gd2v;
 // neighbour exchange across the 64 lanes by DPP wave shifts (VALU moves, no
 // LDS round trip): lane i receives lane i-1 (from_west) or lane i+1
-// (from_east); the end lanes keep their own value, as __shfl_up/down do
+// (from_east); the end lanes, whose levels from the second on are halo, zero
 __device__ inline double from_west(double x)
 {
-  const int lo = __builtin_amdgcn_update_dpp(__double2loint(x), __double2loint(x), 0x138, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(x), __double2hiint(x), 0x138, 0xf, 0xf, false);
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x138, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x138, 0xf, 0xf, true);
   return __hiloint2double(hi, lo);
 }
 __device__ inline double from_east(double x)
 {
-  const int lo = __builtin_amdgcn_update_dpp(__double2loint(x), __double2loint(x), 0x130, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(x), __double2hiint(x), 0x130, 0xf, 0xf, false);
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x130, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x130, 0xf, 0xf, true);
   return __hiloint2double(hi, lo);
 }
 
@@ -115,15 +115,22 @@ __device__ inline void gstore(gdouble* p, const double* v, int cpl)
 // re-read into a scalar register every row step through an empty asm, so the
 // compiler cannot hoist the K x CPL products T1*sx out of the march: they
 // would hold 4K more VGPRs, which at K = 5 costs a wavefront per SIMD.
-// CLDS: the stage coefficients (5 per level, with T1 and T2) are read from
-// LDS (lc[8m + k]) at every row step instead of being held in scalar
-// registers for the whole march, where K = 5 spills 46 of them to vector
-// lanes (read back by v_readlane on the VALU at every use).
-typedef __attribute__((address_space(3))) const double lcdouble;
+// RING: the Y_n and F_n rows, which level m needs m - 1 row steps after they were
+// loaded, wait in LDS (a ring of K - 1 rows per wavefront, every lane its own
+// words, so no barrier) instead of in 8(K - 1) VGPRs, and the stage coefficients
+// are read again at every row step, through the scalar cache, where K = 5 held in
+// scalar registers spills 46 of them to vector lanes.  With the manufactured
+// problem's coefficients as constants that is 123 VGPRs at K = 5 and 138 at K = 6,
+// four and three wavefronts per SIMD, instead of 168 and more than 200, three and
+// two: at 4096^2 35.3 us per stage (39.9 before), 3000^2 21.2 (27.0), 2049^2 15.5
+// (17.6).  The pass is then bound by HBM: at 4096^2, K = 6, its 58 bytes per cell
+// (32 read with the halo, 16 written) move at 4.6 TB/s, a large copy at 4.8.
+typedef __attribute__((address_space(3))) double ldouble;
+typedef __attribute__((address_space(3))) d2v ld2v;
 
-template <int CPL, bool PER, bool MMS, int K, int L, bool FUSED, bool NT, bool SCALAR_E = false, bool CLDS = false>
+template <int CPL, bool PER, bool MMS, int K, int L, bool FUSED, bool NT, bool SCALAR_E = false, bool RING = false>
 __device__ __forceinline__ void pass_wave(const PassGeo& g, const StageEntry* __restrict__ e,
-                                          int strip, int rb, lcdouble* __restrict__ lc = nullptr)
+                                          int strip, int rb, ldouble* ring = nullptr)
 {
   static_assert(K >= 1 && K <= kMaxPassStages, "1..6 stages per pass");
   static_assert(L * CPL >= K - 1, "halo lanes must cover the shrinking levels");
@@ -140,11 +147,18 @@ __device__ __forceinline__ void pass_wave(const PassGeo& g, const StageEntry* __
   const bool he_ok = map_index<PER>(c + CPL, nx, he);
   const bool ld_w = (lane == 0) && hw_ok, ld_e = (lane == kWave - 1) && he_ok;
 
+  // the manufactured problem's coefficients are constants: cell() with the x
+  // products shared between neighbours and the diagonal kept
+  constexpr bool CC = MMS;
+  const double cfx = CC ? ((ccdouble*)g.fx)[0] : 0.0, cfy = CC ? ((ccdouble*)g.fy)[0] : 0.0;
+  const double mdiag = -((cfx + cfx) + (cfy + cfy));
   double Dw0 = 0.0, De0 = 0.0, De1 = 0.0, sx0 = 0.0, sx1 = 0.0, cx0 = 0.0, cx1 = 0.0;
   if (in) {
-    Dw0 = g.fx[cw];
-    De0 = g.fx[cw + 1];
-    if (CPL == 2) De1 = g.fx[cw + 2];
+    if (!CC) {
+      Dw0 = g.fx[cw];
+      De0 = g.fx[cw + 1];
+      if (CPL == 2) De1 = g.fx[cw + 2];
+    }
     if (MMS) {
       sx0 = g.sx[cw];
       cx0 = g.cx[cw];
@@ -154,14 +168,14 @@ __device__ __forceinline__ void pass_wave(const PassGeo& g, const StageEntry* __
       }
     }
   }
-  constexpr int KC = CLDS ? 1 : K;  // coefficient registers (CLDS: unused)
+  constexpr int KC = RING ? 1 : K;  // coefficient registers (RING: unused)
   double cc[KC][5], T1[KC], T2[KC];
 #pragma unroll
   for (int m = 0; m < KC; m++) {
 #pragma unroll
-    for (int k = 0; k < 5; k++) cc[m][k] = (FUSED && !CLDS) ? e[m].c[k] : 0.0;
-    T1[m] = CLDS ? 0.0 : e[m].T1;
-    T2[m] = CLDS ? 0.0 : e[m].T2;
+    for (int k = 0; k < 5; k++) cc[m][k] = (FUSED && !RING) ? e[m].c[k] : 0.0;
+    T1[m] = RING ? 0.0 : e[m].T1;
+    T2[m] = RING ? 0.0 : e[m].T2;
   }
   gcdouble* __restrict__ y0 = (gcdouble*)e[0].yjm1;
   gcdouble* __restrict__ ym = (gcdouble*)e[0].yjm2;
@@ -197,14 +211,44 @@ __device__ __forceinline__ void pass_wave(const PassGeo& g, const StageEntry* __
   const int64_t ts = j0 - (K - 1), te = j1 + (K - 2);  // rows of level 1
 
   double W[K][3][CPL];  // levels 0..K-1: rows south, centre, north
-  double YN[K][CPL], FN[K][CPL];
+  // Y_n and F_n of the last K rows; RING: of this row, the others in the ring
+  constexpr int KR = RING ? 1 : K;
+  double YN[KR][CPL], FN[KR][CPL];
 #pragma unroll
   for (int m = 0; m < K; m++)
 #pragma unroll
     for (int k = 0; k < CPL; k++) {
       W[m][0][k] = W[m][1][k] = W[m][2][k] = 0.0;
-      YN[m][k] = FN[m][k] = 0.0;
+      if (m < KR) YN[m][k] = FN[m][k] = 0.0;
     }
+  // slot s of the ring: Y_n, then F_n, of the 64 lanes
+  constexpr int kRing = RING && FUSED ? K - 1 : 0, kSlot = 2 * kWave * CPL;
+  auto ring_ld = [&](int slot, double* y, double* f) {
+    ldouble* p = ring + slot * kSlot + lane * CPL;
+    if (CPL == 2) {
+      const d2v a = *(ld2v*)p, b = *(ld2v*)(p + kWave * CPL);
+      y[0] = a.x;
+      y[CPL - 1] = a.y;
+      f[0] = b.x;
+      f[CPL - 1] = b.y;
+    } else {
+      y[0] = p[0];
+      f[0] = p[kWave];
+    }
+  };
+  auto ring_st = [&](int slot, const double* y, const double* f) {
+    ldouble* p = ring + slot * kSlot + lane * CPL;
+    if (CPL == 2) {
+      *(ld2v*)p = d2v{y[0], y[CPL - 1]};
+      *(ld2v*)(p + kWave * CPL) = d2v{f[0], f[CPL - 1]};
+    } else {
+      p[0] = y[0];
+      p[kWave] = f[0];
+    }
+  };
+  int head = 0;  // the slot of row t: the ring's oldest row until level K has read it
+#pragma unroll
+  for (int i = 0; i < kRing; i++) ring_st(i, YN[0], FN[0]);  // (zero: rows no owned cell depends on)
   ld_row(y0, ts - 1, W[0][1], false);
   ld_row(y0, ts, W[0][2], false);
   double PR[CPL], PA[CPL], PY[CPL], PG[CPL], Pw, Pe;
@@ -217,7 +261,10 @@ __device__ __forceinline__ void pass_wave(const PassGeo& g, const StageEntry* __
   }
 
   for (int64_t t = ts; t <= te; t++) {
-    if (CLDS) asm volatile("" ::: "memory");  // the coefficients are read again at every row step
+    // RING: the coefficients are read again at every row step
+    typedef __attribute__((address_space(4))) const StageEntry ccentry;
+    ccentry* es = (ccentry*)e;
+    if (RING) asm volatile("" : "+s"(es));
     double A1[CPL];
 #pragma unroll
     for (int k = 0; k < CPL; k++) {
@@ -229,7 +276,7 @@ __device__ __forceinline__ void pass_wave(const PassGeo& g, const StageEntry* __
     const double we = Pw, ee = Pe;
     if (FUSED) {
 #pragma unroll
-      for (int m = K - 1; m > 0; m--)
+      for (int m = KR - 1; m > 0; m--)
 #pragma unroll
         for (int k = 0; k < CPL; k++) {
           YN[m][k] = YN[m - 1][k];
@@ -241,7 +288,7 @@ __device__ __forceinline__ void pass_wave(const PassGeo& g, const StageEntry* __
         FN[0][k] = PG[k];
       }
     }
-    if (t < te) {  // operands of the next iteration
+    if (t < te) {  // operands of the next step
       ld_row(y0, t + 2, PR, false);
       ld_edges(t + 1, Pw, Pe);
       if (FUSED) {
@@ -256,11 +303,29 @@ __device__ __forceinline__ void pass_wave(const PassGeo& g, const StageEntry* __
       const double* S = W[m - 1][0];
       const double* C = W[m - 1][1];
       const double* N = W[m - 1][2];
-      double wv = from_west(C[CPL - 1]);
-      double ev = from_east(C[0]);
+      double pc0 = C[0], pc1 = C[CPL - 1];  // CC: times the x coefficient, with the neighbours'
+      if (CC) {
+        pc0 = cfx * C[0];
+        pc1 = cfx * C[CPL - 1];
+      }
+      double wv = from_west(pc1);
+      double ev = from_east(pc0);
       if (m == 1) {
-        if (lane == 0) wv = we;
-        if (lane == kWave - 1) ev = ee;
+        if (lane == 0) wv = CC ? cfx * we : we;
+        if (lane == kWave - 1) ev = CC ? cfx * ee : ee;
+      }
+      double yv[CPL], gv[CPL];  // Y_n, F_n of the level's row
+      if (FUSED) {
+        if (RING && m > 1) {
+          const int slot = head - (m - 1);
+          ring_ld(slot < 0 ? slot + kRing : slot, yv, gv);
+        } else {
+#pragma unroll
+          for (int k = 0; k < CPL; k++) {
+            yv[k] = YN[RING ? 0 : m - 1][k];
+            gv[k] = FN[RING ? 0 : m - 1][k];
+          }
+        }
       }
       int64_t rw;
       const bool rok = map_index<PER>(rho, ny, rw);
@@ -268,17 +333,27 @@ __device__ __forceinline__ void pass_wave(const PassGeo& g, const StageEntry* __
 #pragma unroll
       for (int k = 0; k < CPL; k++) f[k] = 0.0;
       // wavefront-uniform row coefficients, read before the lane test
-      const double Ds = rok ? fy[rw] : 0.0, Dn = rok ? fy[rw + 1] : 0.0;
+      const double Ds = (!CC && rok) ? fy[rw] : 0.0, Dn = (!CC && rok) ? fy[rw + 1] : 0.0;
       const double syj = (MMS && rok) ? sy[rw] : 0.0, cyj = (MMS && rok) ? cy[rw] : 0.0;
       if (rok && in) {
-        if (CPL == 2) {
+        if (CC) {
+#pragma unroll
+          for (int k = 0; k < CPL; k++) {
+            double x = mdiag * C[k];
+            x = x + (k > 0 ? pc0 : wv);
+            x = x + (k < CPL - 1 ? pc1 : ev);
+            x = x + cfy * S[k];
+            x = x + cfy * N[k];
+            f[k] = 0.0 + x;
+          }
+        } else if (CPL == 2) {
           f[0] = cell(Dw0, De0, Ds, Dn, C[0], wv, C[CPL - 1], S[0], N[0]);
           f[CPL - 1] = cell(De0, De1, Ds, Dn, C[CPL - 1], C[0], ev, S[CPL - 1], N[CPL - 1]);
         } else f[0] = cell(Dw0, De0, Ds, Dn, C[0], wv, ev, S[0], N[0]);
         if (MMS) {
-          double t1 = CLDS ? lc[8 * (m - 1) + 5] : T1[CLDS ? 0 : m - 1];
-          const double t2 = CLDS ? lc[8 * (m - 1) + 6] : T2[CLDS ? 0 : m - 1];
-          if (SCALAR_E && !CLDS) asm volatile("" : "+s"(t1));
+          double t1 = RING ? es[m - 1].T1 : T1[RING ? 0 : m - 1];
+          const double t2 = RING ? es[m - 1].T2 : T2[RING ? 0 : m - 1];
+          if (SCALAR_E && !RING) asm volatile("" : "+s"(t1));
           f[0] = f[0] + forcing(t1, t2, sx0, cx0, syj, cyj);
           if (CPL == 2) f[CPL - 1] = f[CPL - 1] + forcing(t1, t2, sx1, cx1, syj, cyj);
         }
@@ -286,9 +361,9 @@ __device__ __forceinline__ void pass_wave(const PassGeo& g, const StageEntry* __
           const double* Am = (m == 1) ? A1 : W[m >= 2 ? m - 2 : 0][0];
           double cm[5];
 #pragma unroll
-          for (int k = 0; k < 5; k++) cm[k] = CLDS ? lc[8 * (m - 1) + k] : cc[CLDS ? 0 : m - 1][k];
+          for (int k = 0; k < 5; k++) cm[k] = RING ? es[m - 1].c[k] : cc[RING ? 0 : m - 1][k];
 #pragma unroll
-          for (int k = 0; k < CPL; k++) f[k] = lc5(cm, f[k], Am[k], YN[m - 1][k], C[k], FN[m - 1][k]);
+          for (int k = 0; k < CPL; k++) f[k] = lc5(cm, f[k], Am[k], yv[k], C[k], gv[k]);
         }
       }
       if (own && rho >= j0 && rho < j1 && (m == K || m == K - 1))
@@ -301,6 +376,10 @@ __device__ __forceinline__ void pass_wave(const PassGeo& g, const StageEntry* __
           W[m < K ? m : 0][2][k] = f[k];
         }
       }
+    }
+    if (kRing > 0) {
+      ring_st(head, YN[0], FN[0]);
+      head = head + 1 == kRing ? 0 : head + 1;
     }
   }
 }
@@ -333,19 +412,12 @@ __device__ __forceinline__ void axpy_wave(const PassGeo& g, const StageEntry* __
 }
 
 // ---------------------------------------------------------- one problem
-template <int CPL, bool PER, bool MMS, int K, bool NT, bool CLDS>
-__global__ __launch_bounds__(kBlock) void k_pass(const PassGeo g, const StageEntry* __restrict__ e)
+template <int CPL, bool PER, bool MMS, int K, bool NT, bool RING>
+__global__ __launch_bounds__(kBlock, RING && MMS && K <= 5 ? 4 : 1) void k_pass(const PassGeo g, const StageEntry* __restrict__ e)
 {
   constexpr int L = (K - 1 + CPL - 1) / CPL;
-  __shared__ double scoef[CLDS ? 8 * K : 1];
-  if (CLDS) {  // every wavefront of the workgroup reads the same table
-    const int i = threadIdx.x;
-    if (i < 8 * K) {
-      const int m = i >> 3, k = i & 7;
-      scoef[i] = k < 5 ? e[m].c[k] : (k == 5 ? e[m].T1 : (k == 6 ? e[m].T2 : 0.0));
-    }
-    __syncthreads();
-  }
+  constexpr int kRingWave = (K - 1) * 2 * kWave * CPL;  // the wavefront's ring of Y_n and F_n rows
+  __shared__ __attribute__((aligned(16))) double ring[RING && K > 1 ? kWavesPerBlock * kRingWave : 2];
   // XCD-aware: the 8 XCDs receive workgroups round-robin, so workgroup b is
   // given tile (b mod 8)*ceil(T/8) + (b div 8) and each XCD sweeps a
   // contiguous band of row blocks (their halo rows stay in its L2)
@@ -357,7 +429,8 @@ __global__ __launch_bounds__(kBlock) void k_pass(const PassGeo g, const StageEnt
   const int64_t nrb = (g.ny + g.rows - 1) / g.rows;
   if (wt >= (int64_t)g.strips * nrb) return;
   const int strip = (int)(wt % g.strips), rb = (int)(wt / g.strips);
-  pass_wave<CPL, PER, MMS, K, L, true, NT, true, CLDS>(g, e, strip, rb, (lcdouble*)scoef);
+  pass_wave<CPL, PER, MMS, K, L, true, NT, true, RING>(g, e, strip, rb,
+                                                       (ldouble*)ring + (RING ? wave * kRingWave : 0));
 }
 
 PassGeo geo_of(const DiffusionProblem* P, int cpl, int L, int rows)
@@ -377,28 +450,37 @@ PassGeo geo_of(const DiffusionProblem* P, int cpl, int L, int rows)
   return g;
 }
 
-// variant: bit 0 non-temporal operand streams, bit 1 stage coefficients in LDS
-template <int CPL, bool PER, bool MMS>
-void launch_pass_t(const PassGeo& g, int K, int variant, const StageEntry* e, hipStream_t s)
+// the kernel of a K-stage pass; variant: bit 0 non-temporal operand streams,
+// bit 1 RING
+typedef void (*PassKernel)(const PassGeo, const StageEntry*);
+template <int CPL, bool PER, bool MMS, int K>
+PassKernel pass_kernel_k(int variant)
 {
-  const int64_t waves = (int64_t)g.strips * ((g.ny + g.rows - 1) / g.rows);
-  const unsigned grid = (unsigned)((waves + kWavesPerBlock - 1) / kWavesPerBlock);
-#define CEDA_PASS(KK)                                                                                     \
-  switch (variant & 3) {                                                                                  \
-    case 0: hipLaunchKernelGGL((k_pass<CPL, PER, MMS, KK, false, false>), dim3(grid), dim3(kBlock), 0, s, g, e); break; \
-    case 1: hipLaunchKernelGGL((k_pass<CPL, PER, MMS, KK, true, false>), dim3(grid), dim3(kBlock), 0, s, g, e); break;  \
-    case 2: hipLaunchKernelGGL((k_pass<CPL, PER, MMS, KK, false, true>), dim3(grid), dim3(kBlock), 0, s, g, e); break;  \
-    default: hipLaunchKernelGGL((k_pass<CPL, PER, MMS, KK, true, true>), dim3(grid), dim3(kBlock), 0, s, g, e); break; \
+  switch (variant & 3) {
+  case 0: return k_pass<CPL, PER, MMS, K, false, false>;
+  case 1: return k_pass<CPL, PER, MMS, K, true, false>;
+  case 2: return k_pass<CPL, PER, MMS, K, false, true>;
+  default: return k_pass<CPL, PER, MMS, K, true, true>;
   }
+}
+template <int CPL, bool PER, bool MMS>
+PassKernel pass_kernel_t(int K, int variant)
+{
   switch (K) {
-    case 1: CEDA_PASS(1) break;
-    case 2: CEDA_PASS(2) break;
-    case 3: CEDA_PASS(3) break;
-    case 4: CEDA_PASS(4) break;
-    case 5: CEDA_PASS(5) break;
-    default: CEDA_PASS(6) break;
+  case 1: return pass_kernel_k<CPL, PER, MMS, 1>(variant);
+  case 2: return pass_kernel_k<CPL, PER, MMS, 2>(variant);
+  case 3: return pass_kernel_k<CPL, PER, MMS, 3>(variant);
+  case 4: return pass_kernel_k<CPL, PER, MMS, 4>(variant);
+  case 5: return pass_kernel_k<CPL, PER, MMS, 5>(variant);
+  default: return pass_kernel_k<CPL, PER, MMS, 6>(variant);
   }
-#undef CEDA_PASS
+}
+int pass_cpl(const DiffusionProblem* P) { return (P->p.nx % 2 == 0) ? 2 : 1; }
+PassKernel pass_kernel(const DiffusionProblem* P, int K, int variant)
+{
+  const bool per = (P->p.kind == DIFFUSION_CEDA_PERIODIC);
+  if (pass_cpl(P) == 2) return per ? pass_kernel_t<2, true, false>(K, variant) : pass_kernel_t<2, false, true>(K, variant);
+  return per ? pass_kernel_t<1, true, false>(K, variant) : pass_kernel_t<1, false, true>(K, variant);
 }
 
 // ---------------------------------------------------------------- batch
@@ -514,16 +596,24 @@ void launch_pass(DiffusionProblem* P, int K, int rows, int nt, const StageEntry*
   // the kernel reads e[0..K-1]; callers validate K, this keeps a bad one
   // from reaching the device
   if (K < 1 || K > kMaxPassStages || !e || rows < 1) return;
-  const int cpl = (P->p.nx % 2 == 0) ? 2 : 1;
+  const int cpl = pass_cpl(P);
   const PassGeo g = geo_of(P, cpl, pass_halo_lanes(K, cpl), rows);
-  const bool per = (P->p.kind == DIFFUSION_CEDA_PERIODIC);
-  if (cpl == 2) {
-    if (per) launch_pass_t<2, true, false>(g, K, nt, e, s);
-    else launch_pass_t<2, false, true>(g, K, nt, e, s);
-  } else {
-    if (per) launch_pass_t<1, true, false>(g, K, nt, e, s);
-    else launch_pass_t<1, false, true>(g, K, nt, e, s);
-  }
+  const int64_t waves = (int64_t)g.strips * ((g.ny + g.rows - 1) / g.rows);
+  const unsigned grid = (unsigned)((waves + kWavesPerBlock - 1) / kWavesPerBlock);
+  hipLaunchKernelGGL(pass_kernel(P, K, nt), dim3(grid), dim3(kBlock), 0, s, g, e);
+}
+
+// the fewest rows of a tile with which all tiles run in `rounds` rounds of the
+// wavefronts that the GPU holds (a few tiles more take another round)
+int pass_fill_rows(const DiffusionProblem* P, int K, int nt, int rounds)
+{
+  int blocks = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, (const void*)pass_kernel(P, K, nt), kBlock, 0) != hipSuccess)
+    return 0;
+  const int cpl = pass_cpl(P);
+  const PassGeo g = geo_of(P, cpl, pass_halo_lanes(K, cpl), 1);
+  const int64_t fit = (int64_t)blocks * kWavesPerBlock * P->exec->num_cu * rounds / g.strips;  // row blocks
+  return fit < 1 ? 0 : (int)((g.ny + fit - 1) / fit);
 }
 
 void launch_batch_phase(const BatchDesc* desc, const BatchTile* tiles, int ntiles,
