@@ -54,8 +54,30 @@ int call_rhs(ArkMem* A, double t, N_Vector y, N_Vector f)
   return 0;
 }
 
+// whether the vector's operations behind the error weights and the STS error
+// test are the HIP-native ones (an application may replace any of the table):
+// their fused kernels then give the same values
+bool native_error_ops(const ArkMem* A)
+{
+  const N_Vector_Ops o = A->yn->ops;
+  return o->nvabs == N_VAbs_HipNative && o->nvscale == N_VScale_HipNative && o->nvaddconst == N_VAddConst_HipNative &&
+         o->nvinv == N_VInv_HipNative && o->nvlinearcombination == N_VLinearCombination_HipNative &&
+         o->nvwrmsnorm == N_VWrmsNorm_HipNative;
+}
+// whether the error test of an STS step forms the weights itself (a
+// non-positive atol needs their minimum checked)
+bool sts_error_fused(const ArkMem* A)
+{
+  return A->fast || ((A->method == M_RKC || A->method == M_RKL) && A->atol > 0.0 && native_error_ops(A));
+}
+
 int ewt_set(ArkMem* A, N_Vector y)
 {
+  if (A->atol > 0.0 && native_error_ops(A)) {
+    ceda::raw_error_weights(A->rtol, A->atol, y, A->ewt);
+    A->ewt_current = 1;
+    return 0;
+  }
   N_VAbs(y, A->ewt);
   N_VScale(A->rtol, A->ewt, A->ewt);
   N_VAddConst(A->ewt, A->atol, A->ewt);
@@ -415,8 +437,7 @@ void plan_stages(const ArkMem* A, int s, double h, double tn, StagePlan& P)
 int stages_api(ArkMem* A, const StagePlan& P)
 {
   const int s = P.s;
-  N_Vector Yjm2 = A->tv2, Yjm1 = A->tv1, Yj = A->ycur;
-  N_VScale(1.0, A->yn, Yjm2);
+  N_Vector Yjm2 = A->yn, Yjm1 = A->tv1, Yj = A->ycur;
   N_VLinearSum(1.0, A->yn, P.mus1, A->fn, Yjm1);
   double c[5];
   N_Vector X[5];
@@ -427,7 +448,7 @@ int stages_api(ArkMem* A, const StagePlan& P)
     X[0] = Yj; X[1] = Yjm2; X[2] = A->yn; X[3] = Yjm1; X[4] = A->fn;
     if (N_VLinearCombination(5, c, X, Yj)) return ARK_VECTOROP_ERR;
     if (j < s) {
-      N_Vector t = Yjm2;
+      N_Vector t = j == 2 ? A->tv2 : Yjm2;  // (Y_0 is Y_n itself, which stays)
       Yjm2 = Yjm1; Yjm1 = Yj; Yj = t;
     }
   }
@@ -700,9 +721,9 @@ int lsrk_takestep(ArkMem* A, double* dsm)
   r = A->fast ? stages_fused(A, SP) : stages_api(A, SP);
   if (r) return r;
   if (!A->fixedstep) {
-    if (A->fast) {
+    if (sts_error_fused(A)) {
       const double sq = ceda::raw_sts_error_wsqr(
-        A->fast->exec, A->n, N_VGetDeviceArrayPointer(A->yn), N_VGetDeviceArrayPointer(A->ycur),
+        ceda::content(A->yn)->exec, A->n, N_VGetDeviceArrayPointer(A->yn), N_VGetDeviceArrayPointer(A->ycur),
         N_VGetDeviceArrayPointer(A->fn), N_VGetDeviceArrayPointer(A->tv2), h, A->rtol, A->atol);
       *dsm = sqrt(sq / (double)A->n);
     } else {
@@ -1112,7 +1133,7 @@ int step_complete(ArkMem* A, double dsm, double tout, const AttemptState& S)
   A->ycur = t;
   A->nst++;
   A->ewt_current = 0;
-  if (!A->fast && ewt_set(A, A->yn)) return ARK_ILL_INPUT;
+  if (!sts_error_fused(A) && ewt_set(A, A->yn)) return ARK_ILL_INPUT;
   if (!A->fixedstep) {
     const double eta = accept_eta(A, dsm);
     ctrl_update(A, A->h, dsm);

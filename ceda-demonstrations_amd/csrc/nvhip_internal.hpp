@@ -140,6 +140,8 @@ inline unsigned reduce_grid(int64_t n)
   return (unsigned)g;
 }
 
+// ewt = 1/(rtol |y| + atol), as N_VAbs, N_VScale, N_VAddConst, N_VInv
+void raw_error_weights(double rtol, double atol, N_Vector y, N_Vector ewt);
 // raw-pointer helpers used by the integrator's fused STS path; identical
 // arithmetic (and, for the reduction, identical combine order) to the
 // corresponding N_Vector operations
