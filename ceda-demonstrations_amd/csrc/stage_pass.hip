@@ -123,8 +123,8 @@ __device__ inline void gstore(gdouble* p, const double* v, int cpl)
 // problem's coefficients as constants that is 123 VGPRs at K = 5 and 138 at K = 6,
 // four and three wavefronts per SIMD, instead of 168 and more than 200, three and
 // two: at 4096^2 35.3 us per stage (39.9 before), 3000^2 21.2 (27.0), 2049^2 15.5
-// (17.6).  The pass is then bound by HBM: at 4096^2, K = 6, its 58 bytes per cell
-// (32 read with the halo, 16 written) move at 4.6 TB/s, a large copy at 4.8.
+// (17.6).  The pass is then bound by HBM: at 4096^2, K = 6, 50 rows, its 925 MB
+// (counters; 805 without the halo) move at 4.5 TB/s, a large copy at 4.8.
 typedef __attribute__((address_space(3))) double ldouble;
 typedef __attribute__((address_space(3))) d2v ld2v;
 

@@ -58,9 +58,9 @@ int DiffusionProblem_SetStencilRows(DiffusionProblem* prob, int rows);
    streamed operands).  which = 2 is the multi-stage pass of the fused path:
    variant = stages per pass K (2..6; 0 = one kernel per stage), rows = output
    rows per wavefront tile (1..1024), nt a bit mask: 1 non-temporal streamed
-   operands, 2 the stage coefficients read from LDS at every row step instead
-   of held in scalar registers.  Every shape computes bitwise-identical
-   results. */
+   operands, 2 the rows of Y_n and F_n that later stages need kept in LDS and
+   the stage coefficients re-read at every row step, instead of both held in
+   registers.  Every shape computes bitwise-identical results. */
 int DiffusionProblem_SetStencilConfig(DiffusionProblem* prob, int which, int variant, int rows,
                                       int nt);
 int DiffusionProblem_GetStencilConfig(const DiffusionProblem* prob, int which, int* variant,
