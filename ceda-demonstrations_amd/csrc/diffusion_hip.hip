@@ -807,13 +807,19 @@ int DiffusionProblem_Autotune(DiffusionProblem* P, int reps)
   // against 39
   TileCfg bestt;
   float bestt_ms = std::min(best_stage, bestp_ms) * 0.97f;
+  // Small grids, whose tiles leave most CUs idle, are faster on more tiles of
+  // mostly halo, with less work per stage each (adaptive RKC to t = 0.2: 128^2
+  // 3.1 ms with 10 stages on 24 rows, of which a tile owns 2, 3.8 with 8 on 32;
+  // 256^2 5.2 and 6.6); from about 400^2 on they never are
+  const bool small = P->n <= (int64_t)1 << 20;
+  const std::vector<int> waves = small ? std::vector<int>{8, 10, 12, 16} : std::vector<int>{8, 12, 16};
+  const std::vector<int> depths = small ? std::vector<int>{3, 4, 5, 6, 7, 8, 9, 10, 12} : std::vector<int>{3, 4, 6, 8, 10, 12};
   for (int R : {1, 2, 4})
-    for (int nw : {8, 12, 16})
-      for (int K : {3, 4, 6, 8, 10, 12}) {
+    for (int nw : waves)
+      for (int K : depths) {
         const TileCfg c{K, R, nw};
-        // the closing RHS of a step takes one halo row more; tiles of mostly
-        // halo are never the fastest
-        if (!tile_ok(P, c, K, 1) || (P->p.ny > R * nw && R * nw < 3 * (K + 1))) continue;
+        // the closing RHS of a step takes one halo row more
+        if (!tile_ok(P, c, K, 1) || (!small && P->p.ny > R * nw && R * nw < 3 * (K + 1))) continue;
         TileOps o{};
         o.yjm1 = buf[0];
         o.yjm2 = buf[1];

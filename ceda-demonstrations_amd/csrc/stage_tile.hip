@@ -25,7 +25,8 @@
 // 12.0 us (14.8).  The adaptive RKC solve at 128^2 to t = 1 (560 steps of 19
 // right-hand sides) went from 49.9 to 29.5 ms, and to 27.9 ms with the products
 // of constant coefficients shared between cells (tile_stage_cc), which takes
-// 256 uneven problems in a batch from 593 to 536 ms.
+// 256 uneven problems in a batch from 593 to 536 ms; with more, smaller tiles on
+// small grids (the autotuner's choice) and faster reductions it is 19.8 ms.
 //
 // Every value is formed by cell(), forcing() and lc5() in their order: the
 // result is bitwise that of the single-stage kernels.
