@@ -36,6 +36,7 @@
 #include <cstring>
 #include <mutex>
 #include <random>
+#include <type_traits>
 #include <vector>
 
 #include "diffusion_internal.hpp"
@@ -900,7 +901,35 @@ __global__ __launch_bounds__(kBlock) void k_wgrad(const WGradArgs a)
   bfx4 I;  // identity, as a B operand
 #pragma unroll
   for (int j = 0; j < 4; j++) I[j] = (short)(4 * g + j == n ? 0x3f80 : 0);
-  auto transpose = [&](bfx4 v) { return bf_exact4(__builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v, I, zero4, 0, 0, 0)); };
+  // COUNT blocks at once.  An infinity or NaN times the identity's zeros would
+  // reach every channel of its pixel: then (a sum of the products is not finite
+  // in some lane) the blocks are transposed by shuffles.
+  auto transpose = [&](auto count, const bfx4* v, bfx4* out) {
+    constexpr int COUNT = decltype(count)::value;
+    bfx4 in[COUNT];
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < COUNT; k++) {
+      in[k] = v[k];
+      const fx4 p = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(in[k], I, zero4, 0, 0, 0);
+      sum += (p[0] + p[1]) + (p[2] + p[3]);
+      out[k] = bf_exact4(p);
+    }
+    if (__builtin_expect(__all(__builtin_isfinite(sum)), 1)) return;
+#pragma unroll
+    for (int k = 0; k < COUNT; k++) {
+      const uint2 w = __builtin_bit_cast(uint2, in[k]);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {  // channel n of pixel 4g + j
+        const int from = (n >> 2) * 16 + 4 * g + j;
+        const unsigned lo = __shfl(w.x, from, kWave), hi = __shfl(w.y, from, kWave);
+        out[k][j] = (short)(((n & 2) ? hi : lo) >> (16 * (n & 1)));
+      }
+    }
+  };
+  const std::integral_constant<int, 1> one;
+  const std::integral_constant<int, 6> six;
+  const std::integral_constant<int, COUT == kC ? 4 : 3> row;  // the row of x, and of dY where it is one
   const bfx4 none = {0, 0, 0, 0};
 
   const int wave = blockIdx.x * kWavesPB + (threadIdx.x >> 6);
@@ -915,10 +944,12 @@ __global__ __launch_bounds__(kBlock) void k_wgrad(const WGradArgs a)
     const int y0 = c + seg * kWGradRows * d;
     if (y0 >= ny) continue;  // wavefront-uniform: an empty tail segment of a short chain
     const int px = bx * 16 + n;
-    // channels 4g..4g+3 of pixel (bx, n) shifted by s columns in row y, zero outside
+    // channels 4g..4g+3 of pixel (bx, n) shifted by s columns in row y, zero
+    // outside, and for pixels past the row's end, whose dY is zero, whatever
+    // lies there
     auto ld = [&](const void* p, int y, int s) {
       const int xs = px + s;
-      return (y >= 0 && y < ny && xs >= 0 && xs < nx)
+      return (px < nx && y >= 0 && y < ny && xs >= 0 && xs < nx)
                  ? *reinterpret_cast<const bfx4*>(static_cast<const unsigned short*>(p) + act_off(img + y, bpr, xs, g))
                  : none;
     };
@@ -934,34 +965,35 @@ __global__ __launch_bounds__(kBlock) void k_wgrad(const WGradArgs a)
         }
       return v;
     };
-    auto dy_op = [&](bfx4 raw) { return COUT == kC ? transpose(raw) : raw; };
     auto add_bias = [&](bfx4 v) {
 #pragma unroll
       for (int j = 0; j < 4; j++) bsum += bf2f((unsigned short)v[j]);
     };
     if (CIN == kC) {
-      bfx4 xt[3][3], nx_raw[3], ny_raw;
+      bfx4 xt[3][3], raw[4], got[4], top[6];  // raw: the next row of x, and dY's
 #pragma unroll
-      for (int k = 0; k < 3; k++) {
-        xt[1][k] = transpose(ld(a.x, y0 - d, (k - 1) * d));
-        xt[2][k] = transpose(ld(a.x, y0, (k - 1) * d));
-        nx_raw[k] = ld(a.x, y0 + d, (k - 1) * d);
-      }
-      ny_raw = dy_raw(y0);
+      for (int k = 0; k < 6; k++) top[k] = ld(a.x, y0 + (k / 3 - 1) * d, (k % 3 - 1) * d);
+#pragma unroll
+      for (int k = 0; k < 3; k++) raw[k] = ld(a.x, y0 + d, (k - 1) * d);
+      raw[3] = dy_raw(y0);
+      transpose(six, top, top);
+#pragma unroll
+      for (int k = 0; k < 6; k++) xt[1 + k / 3][k % 3] = top[k];
       for (int m = 0; m < kWGradRows; m++) {
         const int y = y0 + m * d;
         if (y >= ny) break;  // wavefront-uniform
-        const bfx4 at = dy_op(ny_raw);
+        transpose(row, raw, got);
+        const bfx4 at = COUT == kC ? got[3] : raw[3];
 #pragma unroll
         for (int k = 0; k < 3; k++) {
           xt[0][k] = xt[1][k];
           xt[1][k] = xt[2][k];
-          xt[2][k] = transpose(nx_raw[k]);
+          xt[2][k] = got[k];
         }
         if (m + 1 < kWGradRows) {
 #pragma unroll
-          for (int k = 0; k < 3; k++) nx_raw[k] = ld(a.x, y + 2 * d, (k - 1) * d);
-          ny_raw = dy_raw(y + d);
+          for (int k = 0; k < 3; k++) raw[k] = ld(a.x, y + 2 * d, (k - 1) * d);
+          raw[3] = dy_raw(y + d);
         }
         add_bias(at);
 #pragma unroll
@@ -980,10 +1012,11 @@ __global__ __launch_bounds__(kBlock) void k_wgrad(const WGradArgs a)
         bfx4 Bop = none;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-          const int xs = bx * 16 + 4 * g + j + (n % 3 - 1) * d;
-          if (n < 9 && ys >= 0 && ys < ny && xs >= 0 && xs < nx) Bop[j] = (short)d2bf(xin[(img + ys) * nx + xs] * is);
+          const int p = bx * 16 + 4 * g + j, xs = p + (n % 3 - 1) * d;
+          if (n < 9 && p < nx && ys >= 0 && ys < ny && xs >= 0 && xs < nx) Bop[j] = (short)d2bf(xin[(img + ys) * nx + xs] * is);
         }
-        const bfx4 at = dy_op(raw);
+        bfx4 at = raw;
+        if (COUT == kC) transpose(one, &raw, &at);
         add_bias(at);
         acc[0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(at, Bop, acc[0], 0, 0, 0);
       }
