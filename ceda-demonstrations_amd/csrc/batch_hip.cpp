@@ -75,6 +75,7 @@ struct DiffusionBatch {
   // large for the last-level cache, where the marching pass is faster (4096^2:
   // 39 against 63 us per stage)
   bool tiles = false, tiles_ok = true;
+  bool marching_set = false;  // thin phases or stages per pass were set: no register tiles from then on
   std::vector<ceda::TileSlot> geo;  // per problem: the constant part of its slots
   unsigned char *d_stage = nullptr, *h_stage = nullptr;  // a group's slots, tiles, coefficients (h pinned)
   size_t cap_stage = 0;
@@ -704,7 +705,7 @@ int DiffusionBatch_SetTileRows(DiffusionBatch* B, int rows)
 {
   if (!B || rows < 0 || rows > 256) return ARK_ILL_INPUT;
   B->tile_rows = rows;
-  use_tiles(B, rows == 0);
+  use_tiles(B, rows == 0 && !B->marching_set);
   if (rows > 0) {
     for (BProb& b : B->probs) set_geometry(b, rows);
     upload_desc(B);
@@ -718,6 +719,7 @@ int DiffusionBatch_SetThinPhases(DiffusionBatch* B, int rows, int min_tiles)
   if (!B || rows < 0 || rows > 256 || min_tiles < 1) return ARK_ILL_INPUT;
   B->thin_rows = rows;
   B->thin_tiles = min_tiles;
+  B->marching_set = true;
   use_tiles(B, false);
   if (B->tuned) upload_desc(B);
   return 0;
@@ -727,6 +729,7 @@ int DiffusionBatch_SetStagesPerPass(DiffusionBatch* B, int kpass)
 {
   if (!B || kpass < 1 || kpass > ceda::kBatchMaxK) return ARK_ILL_INPUT;
   B->kpass = kpass;
+  B->marching_set = true;
   use_tiles(B, false);
   if (!B->tile_rows) B->tuned = false;
   return 0;

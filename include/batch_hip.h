@@ -34,8 +34,10 @@ int DiffusionBatch_SetController(DiffusionBatch* B, int controller);    /* ARK_A
 int DiffusionBatch_SetMaxNumStages(DiffusionBatch* B, int smax);
 int DiffusionBatch_SetMaxNumSteps(DiffusionBatch* B, long mxsteps);
 int DiffusionBatch_SetFixedStep(DiffusionBatch* B, sunrealtype h);
-/* The stage loops run on register tiles unless one of the next three is called
-   with other than SetTileRows(B, 0); the results do not depend on it.
+/* The stage loops run on register tiles unless one of the next three is called:
+   SetThinPhases and SetStagesPerPass choose the marching kernels for good,
+   SetTileRows(B, rows > 0) until SetTileRows(B, 0).  The results do not depend
+   on it.
 
    tile height of the marching kernels: each wavefront tile is `rows` rows of a
    124-column strip (62 for odd nx); rows 1..256, 0 = choose per size class by
