@@ -458,9 +458,12 @@ TileGeo tile_geo(const DiffusionProblem* P, const TileCfg& t, int H)
   return g;
 }
 
+int64_t tile_blocks(const TileGeo& g) { return g.strips * ((g.ny + g.own - 1) / g.own); }
+
 }  // namespace
 
-// a pass of K stages (and the closing RHS) can run on tiles of this shape
+// a pass of K stages (and the closing RHS) can run on tiles of this shape (one
+// of fewer stages then can too)
 bool tile_ok(const DiffusionProblem* P, const TileCfg& t, int K, int rhs)
 {
   if (K < 1 || K > kTileMaxK) return false;
@@ -468,14 +471,17 @@ bool tile_ok(const DiffusionProblem* P, const TileCfg& t, int K, int rhs)
   const int H = K + (rhs ? 1 : 0);
   if (P->p.nx > (int64_t)1 << 30 || P->p.ny > (int64_t)1 << 30) return false;
   const TileGeo g = tile_geo(P, t, H);
-  return g.own >= 1 && 2 * g.hl < kWave;
+  if (g.own < 1 || 2 * g.hl >= kWave) return false;
+  // a launch has fewer than 2^32 threads: few rows per tile on a very tall grid
+  // (2 x 14,000,000 on tiles that own one row) would have more
+  return tile_blocks(g) <= (int64_t)0xffffffff / (t.nw * kWave);
 }
 
 void launch_tile(DiffusionProblem* P, const TileCfg& t, const TileOps& o, hipStream_t s)
 {
-  if (!tile_ok(P, t, o.K, o.rhs)) return;  // callers check; nothing else may reach the kernel
+  if (!tile_ok(P, t, o.K, o.rhs)) CEDA_HIP_CHECK(hipErrorInvalidConfiguration);  // (callers check)
   const TileGeo g = tile_geo(P, t, o.K + (o.rhs ? 1 : 0));
-  const unsigned grid = (unsigned)((int64_t)g.strips * ((g.ny + g.own - 1) / g.own));
+  const unsigned grid = (unsigned)tile_blocks(g);
   const unsigned nt = (unsigned)(t.nw * kWave);
   const size_t lds = sizeof(double2) * 2 * 2 * kWave * (size_t)t.nw;  // at most 64 KiB
   const bool per = P->p.kind == DIFFUSION_CEDA_PERIODIC;
