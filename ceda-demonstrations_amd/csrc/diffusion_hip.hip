@@ -734,6 +734,30 @@ int DiffusionProblem_Autotune(DiffusionProblem* P, int reps)
   hipEvent_t e0, e1;
   CEDA_HIP_CHECK(hipEventCreate(&e0));
   CEDA_HIP_CHECK(hipEventCreate(&e1));
+  // The time of `reps` launches of a pass whose kernel has run before, `par`
+  // being the time of the best shape so far.  One launch tells a shape that is
+  // behind it (most are: a pass over tall tiles of a small grid takes ten times
+  // as long) and saves the others; 20 us are allowed for the host's part in a
+  // single launch, and a short one is tried twice, in case it was interrupted.
+  // With every shape measured in full tuning took 62 ms at 128^2, 244 at
+  // 4096^2 and 803 at 8192^2; now 36, 181 and 565.
+  auto timed = [&](int n, auto&& launch) {
+    float ms = 0.0f;
+    CEDA_HIP_CHECK(hipEventRecord(e0, s));
+    for (int r = 0; r < n; r++) launch();
+    CEDA_HIP_CHECK(hipEventRecord(e1, s));
+    CEDA_HIP_CHECK(hipEventSynchronize(e1));
+    CEDA_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+    return ms;
+  };
+  auto pass_ms = [&](float par, auto&& launch) {
+    const float worst = 1.1f * par + 0.02f * (float)reps, brief = 0.1f * (float)reps;
+    float one = timed(1, launch) * (float)reps;
+    if (one > worst && one < brief) one = timed(1, launch) * (float)reps;
+    if (one > worst) return one;
+    if (one < brief) launch();  // the device is busy when the first timed one is issued
+    return timed(reps, launch);
+  };
   std::vector<StencilCfg> cands;
   for (int rows : {1, 2, 4, 8}) cands.push_back(StencilCfg{0, rows, 0});
   for (int rows : {4, 8, 16, 32, 64})
@@ -783,13 +807,9 @@ int DiffusionProblem_Autotune(DiffusionProblem* P, int reps)
       }
       for (int rows : heights) {
         if (rows > 2 * P->p.ny) continue;
-        launch_pass(P, K, rows, nt, dtab, s);
-        CEDA_HIP_CHECK(hipEventRecord(e0, s));
-        for (int r = 0; r < reps; r++) launch_pass(P, K, rows, nt, dtab, s);
-        CEDA_HIP_CHECK(hipEventRecord(e1, s));
-        CEDA_HIP_CHECK(hipEventSynchronize(e1));
-        float ms = 0.0f;
-        CEDA_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+        auto launch = [&] { launch_pass(P, K, rows, nt, dtab, s); };
+        if (rows == heights[0]) launch();
+        const float ms = pass_ms(bestp_ms * K, launch);
         if (ms / K < bestp_ms) {
           bestp_ms = ms / K;
           bestp = StencilCfg{K, rows, nt};
@@ -806,7 +826,10 @@ int DiffusionProblem_Autotune(DiffusionProblem* P, int reps)
   // arrays come from HBM for every pass and the tiles' halos with them, 63
   // against 39
   TileCfg bestt;
-  float bestt_ms = std::min(best_stage, bestp_ms) * 0.97f;
+  // (a tie goes to the tiles, whose passes also form stage 1 and the closing
+  // RHS: 2999 x 3001 22.5 us per stage either way, a step of 40 stages 1.08 ms
+  // on tiles and 1.29 on k_pass)
+  float bestt_ms = std::min(best_stage, bestp_ms);
   // Small grids, whose tiles leave most CUs idle, are faster on more tiles of
   // mostly halo, with less work per stage each (adaptive RKC to t = 0.2: 128^2
   // 3.1 ms with 10 stages on 24 rows, of which a tile owns 2, 3.8 with 8 on 32;
@@ -814,6 +837,7 @@ int DiffusionProblem_Autotune(DiffusionProblem* P, int reps)
   const bool small = P->n <= (int64_t)1 << 20;
   const std::vector<int> waves = small ? std::vector<int>{8, 10, 12, 16} : std::vector<int>{8, 12, 16};
   const std::vector<int> depths = small ? std::vector<int>{3, 4, 5, 6, 7, 8, 9, 10, 12} : std::vector<int>{3, 4, 6, 8, 10, 12};
+  bool warm[5] = {};
   for (int R : {1, 2, 4})
     for (int nw : waves)
       for (int K : depths) {
@@ -832,13 +856,10 @@ int DiffusionProblem_Autotune(DiffusionProblem* P, int reps)
           for (int k = 0; k < 5; k++) o.c[8 * m + k] = hc[k];
           o.c[8 * m + 6] = 1.0;
         }
-        launch_tile(P, c, o, s);
-        CEDA_HIP_CHECK(hipEventRecord(e0, s));
-        for (int r = 0; r < reps; r++) launch_tile(P, c, o, s);
-        CEDA_HIP_CHECK(hipEventRecord(e1, s));
-        CEDA_HIP_CHECK(hipEventSynchronize(e1));
-        float ms = 0.0f;
-        CEDA_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+        auto launch = [&] { launch_tile(P, c, o, s); };
+        if (!warm[R]) launch();
+        warm[R] = true;
+        const float ms = pass_ms(bestt_ms * K, launch);
         if (ms / K < bestt_ms) {
           bestt_ms = ms / K;
           bestt = c;

@@ -1,0 +1,47 @@
+"""The tuning of a large grid costs about as much as a few thousand of its
+right-hand sides: shapes that one launch shows to be behind are not measured
+further.  4096 x 4098 (a size that no other test tunes): 180 ms, 3,600
+evaluations; with every tile and pass shape measured in full 243 ms, 4,800."""
+import time
+
+import pytest
+
+from hiplib import package
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def pk():
+    return package()
+
+
+@pytest.fixture(scope="module")
+def ctx(pk):
+    c = pk.Context()
+    yield c
+    c.close()
+
+
+def test_tuning_of_a_large_grid(pk, ctx):
+    warm = pk.Problem(ctx, pk.MMS_DIRICHLET, nx=62, ny=58)
+    assert warm.autotune() == 0  # the kernels are loaded
+    G = pk.Problem(ctx, pk.MMS_DIRICHLET, nx=4096, ny=4098)
+    u, f = G.initial(), G.vector()
+    L = pk.lib()
+
+    def rhs_ms(n=400):
+        G.rhs(0.0, u, f)
+        L.N_VMaxNorm(f.h)
+        t = time.perf_counter()
+        for _ in range(n):
+            G.rhs(0.0, u, f)
+        L.N_VMaxNorm(f.h)
+        return (time.perf_counter() - t) * 1e3 / n
+
+    rhs = rhs_ms()
+    t = time.perf_counter()
+    assert G.autotune() == 0
+    tune = (time.perf_counter() - t) * 1e3
+    print("rhs %.4f ms, tuning %.1f ms: %.0f" % (rhs, tune, tune / rhs))
+    assert tune < 4200.0 * rhs
