@@ -23,11 +23,11 @@
 // and the library is built without FMA contraction, which makes the result
 // bitwise identical to a serial CPU evaluation.
 #include <algorithm>
-#include <array>
 #include <cmath>
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <tuple>
 
 #include "diffusion_internal.hpp"
 #include "stencil_ops.hpp"
@@ -414,13 +414,15 @@ void upload_tables(DiffusionProblem* P)
   for (int i = 0; i < nt; i++) *ds[i] = P->d_tables + off[i];
 }
 
-// autotuner results, per (nx, ny, kind) for the life of the process
+// autotuner results for the life of the process: by size, kind and whether the
+// coefficients are constant (the tiles then run another kernel)
 struct TuneKey {
   int64_t nx, ny;
   int kind;
+  bool constant;
   bool operator<(const TuneKey& o) const
   {
-    return nx != o.nx ? nx < o.nx : (ny != o.ny ? ny < o.ny : kind < o.kind);
+    return std::tie(nx, ny, kind, constant) < std::tie(o.nx, o.ny, o.kind, o.constant);
   }
 };
 struct TuneResult {
@@ -710,7 +712,7 @@ extern "C" {
 int DiffusionProblem_Autotune(DiffusionProblem* P, int reps)
 {
   if (!P || reps < 1) return -1;
-  const TuneKey key{P->p.nx, P->p.ny, P->p.kind};
+  const TuneKey key{P->p.nx, P->p.ny, P->p.kind, P->constant_faces};
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tune.find(key);

@@ -73,11 +73,12 @@ int DiffusionProblem_GetStencilConfig(const DiffusionProblem* prob, int which, i
    which = 2 switches them off.  Bitwise the same results. */
 int DiffusionProblem_SetTileConfig(DiffusionProblem* prob, int K, int rows, int waves);
 int DiffusionProblem_GetTileConfig(const DiffusionProblem* prob, int* K, int* rows, int* waves);
-/* times every candidate launch shape of the three kernels on scratch buffers
-   of the problem's size (reps launches each, HIP events) and keeps the
-   fastest; multi-stage passes are enabled only when their time per stage
-   beats the best single-stage kernel.  Results are cached per (nx, ny, kind)
-   for the life of the process */
+/* times the candidate launch shapes of the three kernels and of the register
+   tiles on scratch buffers of the problem's size (HIP events; reps launches
+   each, or one for a pass or tile shape that it shows to be behind) and keeps
+   the fastest; multi-stage passes are enabled only when their time per stage
+   beats the best single-stage kernel.  Results are cached per nx, ny, kind and
+   constant or varying coefficients for the life of the process */
 int DiffusionProblem_Autotune(DiffusionProblem* prob, int reps);
 
 /* [ext] times `reps` back-to-back launches of one hot-path kernel with HIP
