@@ -2610,7 +2610,8 @@ int LearnedPrec_MakeTrainingSetXY(int nsamp, int n, double ratio_x, double ratio
   bool all = false;
   constexpr int kChunk = 256;  // iterations per launch of the one-CU solves (a launch of bounded length)
   while (!all && it < maxit) {
-    if (cg_solve(nsamp, n, ratio_x, ratio_y, idg, reltol * reltol, kChunk, e, tmp, p, st, s)) it += kChunk;
+    const int chunk = std::min(kChunk, maxit - it);
+    if (cg_solve(nsamp, n, ratio_x, ratio_y, idg, reltol * reltol, chunk, e, tmp, p, st, s)) it += chunk;
     else for (int k = 0; k < 50; k++, it++)
       if (n % 2 == 0)
         hipLaunchKernelGGL(k_cg_iter<true>, dim3(nsamp), dim3(kBlock), 0, s, n, ratio_x, ratio_y, idg,
