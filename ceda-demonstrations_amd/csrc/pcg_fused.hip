@@ -26,9 +26,10 @@
 // The scalars never go to the host: every workgroup first sums the previous
 // kernel's per-workgroup partials itself, in one fixed order (every workgroup
 // gets bitwise the same alpha or beta), while its first cells' operands are
-// already being loaded; the residual test is recorded in a device status word
-// (running, converged at iteration l, non-finite) that every later kernel
-// reads first, returning at once when the solve has ended.  The host enqueues
+// already being loaded; the residual test is recorded in the device's solve
+// state (running, converged at iteration l, non-finite), which every later
+// kernel reads first, returning at once when the solve has ended.  The host
+// enqueues
 // iterations in batches, of the previous solve's length at first, and reads
 // the status once per batch (after a one-workgroup kernel has tested the
 // batch's last iteration and written the state to host memory): the iteration
@@ -68,8 +69,11 @@ constexpr int kStateDoubles = 8;
 constexpr int kWsDoubles = kOffState + kStateDoubles;
 
 // solve state in device memory (doubles): r.z of the current iteration in
-// slot l & 1, the status word, the iteration it was set at, the last |r|^2
-enum { kRz0 = 0, kRz1 = 1, kStatus = 2, kIter = 3, kRr = 4, kDelta = 5 };
+// slot l & 1, the status, the iteration it was set at, the last |r|^2 and
+// delta.  The status stands in two words, so that no kernel stores one that
+// its other wavefronts read: k_pcg_dir returns by kStatus and records its test
+// in kTested, k_pcg_update returns by kTested and hands it on to kStatus.
+enum { kRz0 = 0, kRz1 = 1, kStatus = 2, kIter = 3, kRr = 4, kDelta = 5, kTested = 6 };
 enum { kRunning = 0, kConverged = 1, kNonFinite = 2 };
 
 // x of the lanes `CTRL` (DPP) rows or lanes below; zero where there is none
@@ -141,7 +145,7 @@ __device__ inline void sum_partials(const double* __restrict__ partials, int nbl
   }
 }
 
-__device__ inline bool solve_ended(const double* __restrict__ st) { return st[kStatus] != kRunning; }
+__device__ inline bool solve_ended(const double* __restrict__ st, int word = kStatus) { return st[word] != kRunning; }
 
 // Jacobi inverse diagonal from the face coefficients: dinv = 1 / (1 - gp d),
 // d = -((ax[i] + ax[i+1]) + (ay[j] + ay[j+1])), exactly k_psetup's value for
@@ -158,14 +162,14 @@ __device__ inline double jac_dinv(const JacobiDiag& J, double sxi, double syj)
 
 // the residual test of iteration l-1 from k_pcg_update's partials (|r|^2,
 // r.z): converged, non-finite (|r| or beta), else running with
-// beta = r.z(l-1) / r.z(l-2).  Workgroup 0 records the outcome; the caller
-// returns when the solve has ended.
+// beta = r.z(l-1) / r.z(l-2).  Workgroup 0 records the outcome, an end in
+// `word`; the caller returns when the solve has ended.
 // r.z comes from parts_b's second accumulator, or, when parts_z is given
 // (a preconditioner callback computed z after the update), from k_pcg_dot's
 // partials parts_z.
 __device__ inline bool test_iteration(int nparts, const double* __restrict__ parts_b,
-                                      const double* __restrict__ parts_z, double* __restrict__ st, int l,
-                                      double* beta)
+                                      const double* __restrict__ parts_z, double* __restrict__ st, int word,
+                                      int l, double* beta)
 {
   const double rzold = st[(l - 1) & 1], delta = st[kDelta];
   double b2[2], z1[1];
@@ -186,7 +190,7 @@ __device__ inline bool test_iteration(int nparts, const double* __restrict__ par
     st[kRr] = rr;
     st[kIter] = l - 1;
     if (status == kRunning) st[l & 1] = rznew;  // the r.z iteration l uses
-    else st[kStatus] = status;
+    else st[word] = status;
   }
   return status != kRunning;
 }
@@ -320,7 +324,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_dir(const PcgGrid g, double gamm
   }
   const double dz = (ZS == kZConst) ? jac_dinv(J, J.ax[0] + J.ax[1], J.ay[0] + J.ay[1]) : 1.0;
   double beta = 0.0;
-  if (!first && test_iteration(nparts, parts_b, parts_z, st, l, &beta)) return;
+  if (!first && test_iteration(nparts, parts_b, parts_z, st, kTested, l, &beta)) return;
   auto dir = [&](double zv, double pv) { return ((ZS == kZConst) ? dz * zv : zv) + beta * pv; };
   double acc[1] = {0.0};
   while (u.valid()) {
@@ -358,13 +362,16 @@ enum { kUpCallback = 0, kUpConst = 1, kUpNone = 2, kUpJacobi = 3, kUpArray = 4 }
 template <bool PER, int UP, int W>
 __global__ __launch_bounds__(kBlock) void k_pcg_update(const PcgGrid g, double gamma, int nparts,
                                                        const double* __restrict__ parts_a,
-                                                       const double* __restrict__ st, int l,
+                                                       double* __restrict__ st, int l,
                                                        const double* __restrict__ p, double* __restrict__ x,
                                                        double* __restrict__ r, double* __restrict__ z,
                                                        const double* __restrict__ dinv, JacobiDiag J,
                                                        const double* __restrict__ w, double* __restrict__ partials)
 {
-  if (solve_ended(st)) return;
+  if (solve_ended(st, kTested)) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) st[kStatus] = st[kTested];
+    return;
+  }
   UnitWalk<W> u(g);
   Five<W> pv = {};
   double xv[W] = {}, rv[W] = {};
@@ -430,7 +437,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_check(int nparts, const double* 
 {
   if (!solve_ended(st)) {
     double beta;
-    test_iteration(nparts, parts_b, parts_z, st, l, &beta);
+    test_iteration(nparts, parts_b, parts_z, st, kStatus, l, &beta);
   }
   state_to_host(st, host);
 }
@@ -480,7 +487,7 @@ __global__ void k_pcg_init(double* __restrict__ st, double rz, double delta)
   if (threadIdx.x == 0) {
     st[kRz0] = 0.0;
     st[kRz1] = rz;  // iteration 1 reads slot 1
-    st[kStatus] = kRunning;
+    st[kStatus] = st[kTested] = kRunning;
     st[kIter] = 0;
     st[kRr] = 0.0;
     st[kDelta] = delta;
