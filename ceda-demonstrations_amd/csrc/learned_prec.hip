@@ -2332,9 +2332,10 @@ bool launch_cg_solve(int nsamp, int n, double rx, double ry, double idg, double 
 {
   const size_t lds = sizeof(double) * (size_t)std::min(n * n, T * CPL);
   if (lds > 32768) {
-    static const hipError_t allowed = hipFuncSetAttribute(
-        (const void*)k_cg_solve<T, CPT, CPL, W>, hipFuncAttributeMaxDynamicSharedMemorySize, 8 * T * CPL);
-    if (allowed != hipSuccess) {
+    // (an attribute of the current device's kernel: asked at every launch, 256
+    // iterations apart, not once per process)
+    if (hipFuncSetAttribute((const void*)k_cg_solve<T, CPT, CPL, W>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            8 * T * CPL) != hipSuccess) {
       (void)hipGetLastError();
       return false;
     }
