@@ -73,7 +73,7 @@ struct DiffusionBatch {
   // register tiles (stage_tile.hip), unless the caller chose marching tiles
   // (tile rows, thin phases, stages per pass) or most cells are in problems too
   // large for the last-level cache, where the marching pass is faster (4096^2:
-  // 39 against 63 us per stage)
+  // 35 against 63 us per stage)
   bool tiles = false, tiles_ok = true;
   bool marching_set = false;  // thin phases or stages per pass were set: no register tiles from then on
   std::vector<ceda::TileSlot> geo;  // per problem: the constant part of its slots
@@ -412,8 +412,12 @@ void run_marching(DiffusionBatch* B, const std::vector<int>& planned, bool adapt
 // 24 ragged ones to t = 0.01 14 ms, a whole call 112 -> 20 ms, where the marching
 // tiles also timed seven tile heights for every size class.
 constexpr int64_t kTileCells = (int64_t)4 << 20;
-// below this many tiles of 64 rows a pass runs on tiles of 32 rows (own 10
-// rows instead of 42, half the time per tile): the GPU has 256 CUs
+// Up to this many tiles of 64 rows a pass runs on tiles of 32 rows, which own 10
+// rows instead of 42: four times as many, of half the time each, which pays
+// while they find a CU each (there are 256).  A step of 27 stages: one problem
+// of 128^2 (4 tall tiles) 57 us on low tiles, 83 on tall ones; four of 200^2 (40)
+// 72, 103; eight (80) 137, 129; six of 300^2 (144) 160, 124; two of 1000^2 (480)
+// 308, 194.
 constexpr int kTileThin = 64;
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 void run_tiles(DiffusionBatch* B, const std::vector<int>& planned, bool adaptive)

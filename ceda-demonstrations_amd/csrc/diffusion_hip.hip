@@ -826,7 +826,8 @@ int DiffusionProblem_Autotune(DiffusionProblem* P, int reps)
   // 128^2 1.6 against 2.8 us per stage, 777 x 1001 2.2 against 6.6, 2048^2 12.0
   // against 14.8 (periodic 8.8 against 16.8); at 4096^2, where the four operand
   // arrays come from HBM for every pass and the tiles' halos with them, 63
-  // against 39
+  // against 35 (a periodic problem is faster on tiles there too: a step of 40
+  // stages 1.65 ms against 2.13)
   TileCfg bestt;
   // (a tie goes to the tiles, whose passes also form stage 1 and the closing
   // RHS: 2999 x 3001 22.5 us per stage either way, a step of 40 stages 1.08 ms

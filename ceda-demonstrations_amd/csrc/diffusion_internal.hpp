@@ -86,10 +86,13 @@ void launch_rhs_entry(DiffusionProblem* P, const StageEntry* e, hipStream_t s);
 
 // K consecutive fused stages in one sweep (temporal blocking): stages read
 // e[0].yjm1, e[0].yjm2, e[0].yn, e[0].fn; stage K-1 is written to e[K-2].out
-// and stage K to e[K-1].out (K = 1..4).  rows = output rows per wavefront
-// tile, nt = non-temporal streams.  Bitwise equal to K single-stage launches.
-int pass_fill_rows(const DiffusionProblem* P, int K, int nt, int rounds);
+// and stage K to e[K-1].out (K = 1..kMaxPassStages).  rows = output rows per
+// wavefront tile, nt: bit 0 non-temporal streams, bit 1 Y_n and F_n rows in LDS
+// and coefficients re-read.  Bitwise equal to K single-stage launches.
 void launch_pass(DiffusionProblem* P, int K, int rows, int nt, const StageEntry* e, hipStream_t s);
+// the fewest rows with which the pass's tiles run in `rounds` rounds of the
+// wavefronts that the GPU holds (0: unknown)
+int pass_fill_rows(const DiffusionProblem* P, int K, int nt, int rounds);
 // halo lanes of a K-stage pass (each side of a wavefront strip)
 int pass_halo_lanes(int K, int cpl);
 

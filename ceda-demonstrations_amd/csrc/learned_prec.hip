@@ -1563,7 +1563,11 @@ __global__ __launch_bounds__(kBlock) void k_cg_iter(int n, double rx, double ry,
 // cache (257 us, 7.1 TB/s, with all p in memory; 537 us by k_cg_iter), 160^2
 // 87 us, 128^2 32 us (223 by k_cg_iter), 100^2 26 us (140).
 constexpr int kCgLdsSide = 128;   // p in LDS: 128 KiB
-constexpr int kCgRegSide = 192;   // r in registers: 36 cells per thread
+// r in registers: 36 cells per thread, which take 124 of the 128 VGPRs that a
+// thread of 1024 has (40 cells: 14 spilled).  Larger sides are solved by
+// k_cg_iter; 1,024 pairs of 192^2 take 112 ms here, of 194^2 397 ms there, of
+// 193^2 (single cells) 550 ms.
+constexpr int kCgRegSide = 192;
 constexpr int kCgCellsLds = 16;   // cells per thread, p in LDS
 constexpr int kCgCellsMem = 36;   // cells per thread, p partly in memory
 constexpr int kCgCellsHalf = 18;  // of them in LDS: 144 KiB
