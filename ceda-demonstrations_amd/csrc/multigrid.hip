@@ -215,9 +215,9 @@ __global__ __launch_bounds__(kBlock) void k_mg_prolong(const MGLevelD F, const M
 // infinities and NaN, the division's own fix-up: 6 instructions instead of
 // the 13 of a division.  The bits are the division's while d, the diagonal of
 // I - gamma J, is from 1 to 2^50 and n zero, not finite or at least 2^-900;
-// below, where a residual may underflow, the last bits may differ.  (A test for such n at every
-// quotient, or once per pass with the least |n| kept, made a cycle at 2048^2
-// 185 us long instead of 166.)
+// below, where a residual may underflow, the last bits may differ.  (A test for
+// such n at every quotient, or once per pass with the least |n| kept, made a
+// cycle at 2048^2 185 us long instead of 166.)
 __device__ inline double mg_quot(double n, double d, double y)  // n / d, y = 1 / d
 {
   double q = n * y;
